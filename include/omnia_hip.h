@@ -561,6 +561,47 @@ int32_t omnia_attention_decode_noalloc(const uint16_t* raw_queries, const uint16
                                        int64_t head_dim, float scale, float eps, uint16_t* out,
                                        hipStream_t stream);
 
+/* The prologue of an attention layer over `length` tokens: q and k normed per head (where a
+ * gain is given) and rotated by the given angle rows, k and v written into cache rows,
+ *   n = bf16(w * bf16(x * inv)), inv = 1 / sqrt(sum x^2 / D + eps)     (n = x without a gain)
+ *   a, b = bf16(n_p * bf16(mscale)), bf16(n_{p+P} * bf16(mscale))       p < P = rotary_pairs
+ *   y_p = bf16(a cos - b sin), y_{p+P} = bf16(a sin + b cos), y_d = n_d for d >= 2P
+ * raw_queries [length, heads * D], raw_keys / raw_values [length, kv_heads * D], rows their
+ * strides apart; query_weight, key_weight [D] bf16 or null; cos_rows, sin_rows [length, P]
+ * fp32, `table_stride` floats apart, 16-byte aligned (null with P = 0); queries [heads,
+ * length, D]; key_rows and value_rows: head h, token t at h * head_stride + t * D.
+ * Replaces: core/kernels/attention/default.py:85-131 (the norms, the rotation and
+ * `update_and_fetch`'s writes of the Core chain), in one launch.
+ * head_dim 64 or 128; rotary_pairs a multiple of 8 with 2P <= D. */
+int32_t omnia_attention_project(const uint16_t* raw_queries, int64_t query_stride,
+                                const uint16_t* raw_keys, int64_t key_stride,
+                                const uint16_t* raw_values, int64_t value_stride,
+                                const uint16_t* query_weight, const uint16_t* key_weight,
+                                const float* cos_rows, const float* sin_rows, int64_t table_stride,
+                                int64_t rotary_pairs, float mscale, float eps, int64_t length,
+                                int64_t heads, int64_t kv_heads, int64_t head_dim,
+                                uint16_t* queries, uint16_t* key_rows, int64_t key_head_stride,
+                                uint16_t* value_rows, int64_t value_head_stride, hipStream_t stream);
+
+/* Attention of `length` queries per head over `rows` cached rows (the queries are the last
+ * `length` of them):
+ *   s[h, t, r] = scale * (q[h, t] . keys[h / gqa, r]) where r is attended
+ *   out[h, t] = sum_r exp(s - M) values[h / gqa, r] / (exp(sink[h] - M) + sum_r exp(s - M))
+ * in fp32 (the probabilities in full), rounded once to bf16; no sink term with null sinks.
+ * causal = 1: query t attends rows <= rows - length + t; a mask ([length, rows] bytes, rows
+ * `mask_stride` apart, non-zero attends) is applied as well. A query that attends nothing
+ * gives 0 / 0 (0 with a sink). queries, out [heads, length, D]; keys, values: head h, row r
+ * at h * head_stride + r * D.
+ * Replaces: core/kernels/attention/default.py:132-156 (the attention of the Core chain at
+ * T > 1, which a prefill runs).
+ * head_dim 64 or 128; heads a multiple of kv_heads; scale positive and finite. */
+int32_t omnia_attention_prefill(const uint16_t* queries, const uint16_t* keys,
+                                const uint16_t* values, int64_t key_head_stride,
+                                int64_t value_head_stride, int64_t heads, int64_t kv_heads,
+                                int64_t head_dim, int64_t length, int64_t rows, int32_t causal,
+                                const uint8_t* mask, int64_t mask_stride, const uint16_t* sinks,
+                                float scale, uint16_t* out, hipStream_t stream);
+
 /* Calibration copy: dst[0 .. bytes) = src[0 .. bytes), 16-byte nontemporal loads and
  * stores, `vectors_per_thread` (1, 2 or 4) vectors per thread issued before the first
  * store. bytes a multiple of 16; both pointers 16-byte aligned; the ranges must not

@@ -9,14 +9,15 @@ whose `build` accepts it serves the layer.
   reference's `FullAttentionStep` (a fixed cache, core/kernels/attention/full.py:632-740)
   and `SlidingAttentionStep` (a ring, sliding.py:583-691) serve: bf16, head_dim 128,
   q/k norm gains, a rotary table, no sinks; one fused step that writes the new K/V row
-  into the cache and reads the position on the device. A prefill (T != 1) goes to the
-  Core chain, as in the reference.
+  into the cache and reads the position on the device. A prefill (T != 1) runs on the
+  prefill kernels (prefill.py) where they compute it alike, else on the Core chain.
 - `HipSinkAttentionStep` (`omnia_attention_sink_decode`, csrc/attention_sink.hip) serves
   what the reference's `SinkAttentionStep` serves (core/kernels/attention/sink.py:256-366):
   a layer with learned sink logits over a growing `KVCache`, bf16, head_dim 64, 1, 2, 4
-  or 8 query heads per kv head; the norms, the rotation and the cache write run as in the
-  Core chain, then one split-K attention with the sink in the softmax's denominator. A
-  prefill goes to the Core chain, as in the reference.
+  or 8 query heads per kv head; the norms, the rotation and the cache write in one launch
+  (prefill.py `project`, else as in the Core chain), then one split-K attention with the
+  sink in the softmax's denominator. A prefill runs on the prefill kernels, else on the
+  Core chain.
 - `DefaultAttentionStep` is the Core chain (core/kernels/attention/default.py:85-156): the
   norms, the rotation, `cache.update_and_fetch` and attention in torch ops (fp32). It
   accepts everything, sinks included.
@@ -35,6 +36,7 @@ from ..qkv_rope.atlas import AngleAtlas
 from ..qkv_rope.kernel import AngleTable
 from ..resolve import record_fallback, resolve
 from .cache import FixedKVCache, KVCache, RingKVCache
+from .prefill import prefill, project, project_served
 
 __all__ = ["AttentionStep", "AttentionStepStrategy", "DefaultAttentionStep", "FixedKVCache",
            "HipAttentionStep", "HipSinkAttentionStep", "KVCache", "RingKVCache", "attention_step_applies",
@@ -241,6 +243,9 @@ class HipAttentionStep(AttentionStepStrategy):
 
     def __call__(self, raw_queries, raw_keys, raw_values, mask=None):
         if raw_queries.shape[1] != 1:
+            out = prefill(self.fallback, raw_queries, raw_keys, raw_values, mask)
+            if out is not None:
+                return out
             record_fallback(self, self.fallback)
             return self.fallback(raw_queries, raw_keys, raw_values, mask)
         cache = self.cache
@@ -284,9 +289,9 @@ def sink_step_applies(heads: int, kv_heads: int, head_dim: int) -> bool:
 @dataclass(frozen=True)
 class HipSinkAttentionStep(AttentionStepStrategy):
     """The decode step of a layer with learned sinks over a growing `KVCache`: the norms,
-    the rotation and the cache write as the Core chain runs them (the reference's
-    SinkAttentionStep runs them in ops too, core/kernels/attention/sink.py:330-352), then
-    the attention on `omnia_attention_sink_decode`. A prefill goes to the Core chain."""
+    the rotation and the cache write in one launch (the reference's SinkAttentionStep runs
+    them in ops, core/kernels/attention/sink.py:330-352), then the attention on
+    `omnia_attention_sink_decode`."""
 
     core: DefaultAttentionStep
     sinks: torch.Tensor
@@ -308,9 +313,16 @@ class HipSinkAttentionStep(AttentionStepStrategy):
 
     def __call__(self, raw_queries, raw_keys, raw_values, mask=None):
         if raw_queries.shape[1] != 1:
+            out = prefill(self.core, raw_queries, raw_keys, raw_values, mask)
+            if out is not None:
+                return out
             record_fallback(self, self.core)
             return self.core(raw_queries, raw_keys, raw_values, mask)
-        q, keys, values = self.core.project(raw_queries, raw_keys, raw_values)
+        projected = None
+        if project_served(self.core, raw_queries, raw_keys, raw_values):
+            projected = project(self.core, raw_queries, raw_keys, raw_values)
+        q, keys, values = (projected if projected is not None
+                           else self.core.project(raw_queries, raw_keys, raw_values))
         if q.dtype != torch.bfloat16 or not hip_device(q, keys, values):
             raise ValueError("sink attention step: the projections must be bf16 on the sinks' device")
         band = None if isinstance(mask, str) else mask

@@ -1,0 +1,177 @@
+"""A prefill (or one step of a sink layer) on `omnia_attention_project` and
+`omnia_attention_prefill` (csrc/attention_prefill.hip): the norms, the rotation, the cache
+write and the attention that `DefaultAttentionStep` runs in torch ops
+(core/kernels/attention/default.py:85-156), for the calls these kernels compute alike.
+
+`project_served` says whether a call's prologue is one of them, before anything is written:
+plain bf16 tensors of the current ROCm device, head_dim 64 or 128, a cache of this package
+with room, gains and angle rows the kernel can read. A call that autograd, a functorch
+transform, a dispatch mode or a compiler follows stays with the torch ops, which they can
+see through. `mask_served` does the same for the attention's mask.
+"""
+
+from __future__ import annotations
+
+import math
+
+import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
+
+from ...runtime import ops
+from .._device import hip_device
+from ..qkv_rope.atlas import AngleAtlas
+from ..qkv_rope.kernel import AngleTable
+from .cache import FixedKVCache, KVCache
+
+HEAD_DIMS = (64, 128)
+
+
+def plain_call(*tensors: torch.Tensor) -> bool:
+    """Ordinary tensors on the current ROCm device, with nothing following the operations
+    on them: a kernel may then stand in for torch ops."""
+    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0:
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    if any(type(mode) is not DeviceContext for mode in _get_current_function_mode_stack()):
+        return False
+    if torch.autograd.forward_ad._current_level >= 0:
+        return False
+    if any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in tensors):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    return hip_device(*tensors) and tensors[0].device.index == torch.cuda.current_device()
+
+
+def _rows_readable(raw: torch.Tensor, length: int, width: int) -> bool:
+    return raw.dtype == torch.bfloat16 and tuple(raw.shape) == (1, length, width)
+
+
+def _gain_readable(weight: torch.Tensor | None, head_dim: int) -> bool:
+    return weight is None or (weight.dtype == torch.bfloat16 and weight.is_contiguous()
+                              and weight.numel() == head_dim and weight.data_ptr() % 16 == 0)
+
+
+def _cache_writable(cache, length: int, kv_heads: int, head_dim: int) -> bool:
+    """A cache whose rows the prologue may write itself: this package's fixed cache with
+    room, or its growing one, of bf16 rows the kernels read in place."""
+    if type(cache) is FixedKVCache:
+        if cache.offset + length > cache.capacity:
+            return False
+    elif type(cache) is not KVCache:
+        return False
+    for buffer in (cache.keys, cache.values):
+        if buffer is None:
+            continue
+        if (buffer.dtype != torch.bfloat16 or not buffer.is_contiguous() or buffer.dim() != 4
+                or buffer.shape[0] != 1 or buffer.shape[1] != kv_heads or buffer.shape[3] != head_dim
+                or buffer.data_ptr() % 16 != 0):
+            return False
+    return True
+
+
+def project_served(core, raw_queries, raw_keys, raw_values) -> bool:
+    """Whether `project` computes this call's prologue as `core` (a `DefaultAttentionStep`)
+    does."""
+    if raw_queries.dim() != 3 or core.head_dim not in HEAD_DIMS or core.heads % core.kv_heads:
+        return False
+    length, d = raw_queries.shape[1], core.head_dim
+    if length == 0 or not (_rows_readable(raw_queries, length, core.heads * d)
+                           and _rows_readable(raw_keys, length, core.kv_heads * d)
+                           and _rows_readable(raw_values, length, core.kv_heads * d)):
+        return False
+    if core.rotary_pairs % 8 or 2 * core.rotary_pairs > d:
+        return False
+    if not (_gain_readable(core.query_weight, d) and _gain_readable(core.key_weight, d)):
+        return False
+    cache = core.cache
+    if not _cache_writable(cache, length, core.kv_heads, d):
+        return False
+    held = [t for t in (core.query_weight, core.key_weight, core.sinks, getattr(cache, "keys", None),
+                        getattr(cache, "values", None)) if t is not None]
+    return plain_call(raw_queries, raw_keys, raw_values, *held)
+
+
+def mask_served(mask, length: int, rows: int) -> bool:
+    """No mask, a string ("causal", or another, which the Core chain ignores) or a boolean
+    one of a row per query."""
+    if mask is None or isinstance(mask, str):
+        return True
+    return (mask.dtype == torch.bool and tuple(mask.shape) in ((length, rows), (1, length, rows), (1, 1, length, rows))
+            and (rows <= 1 or mask.stride(-1) == 1) and (length <= 1 or mask.stride(-2) >= rows)
+            and plain_call(mask))
+
+
+def _readable_rows(raw: torch.Tensor) -> torch.Tensor:
+    """The [T, width] rows, copied where the kernel could not read them in place."""
+    rows = raw[0]
+    if rows.stride(-1) != 1 or rows.stride(0) % 8 or rows.stride(0) < rows.shape[1] or rows.data_ptr() % 16:
+        rows = rows.clone(memory_format=torch.contiguous_format)
+    return rows
+
+
+def _angle_rows(core, length: int, device):
+    """The (cos, sin) rows of this call's positions, or None where the layer rotates
+    nothing or the table holds too few rows."""
+    offset, pairs = core.cache.offset, core.rotary_pairs
+    if type(core.angles) is AngleTable:
+        cos, sin = core.angles.cos[offset : offset + length], core.angles.sin[offset : offset + length]
+    elif type(core.angles) is AngleAtlas:
+        rows = core.angles(offset, length)
+        cos, sin = rows[:, :pairs], rows[:, pairs : 2 * pairs]
+    else:
+        cos, sin = core._angles(offset, length, device)
+    for rows in (cos, sin):
+        if (rows.dtype != torch.float32 or rows.device != device or tuple(rows.shape) != (length, pairs)
+                or rows.stride(-1) != 1 or rows.data_ptr() % 16 or (length > 1 and rows.stride(0) % 4)
+                or rows.stride(0) != cos.stride(0)):
+            return None
+    return cos, sin
+
+
+def project(core, raw_queries, raw_keys, raw_values):
+    """(queries [heads, T, D], keys, values) as `core.project` gives them, the cache written
+    and advanced; None, with nothing written, where the angle rows cannot be read in place."""
+    length, device = raw_queries.shape[1], raw_queries.device
+    angles = None
+    if core.rotary_pairs:
+        angles = _angle_rows(core, length, device)
+        if angles is None:
+            return None
+    key_rows, value_rows = core.cache.claim(length, core.kv_heads, core.head_dim, raw_keys)
+    queries = ops.attention_project(
+        _readable_rows(raw_queries), _readable_rows(raw_keys), _readable_rows(raw_values),
+        core.query_weight, core.key_weight, angles, key_rows, value_rows, heads=core.heads,
+        kv_heads=core.kv_heads, head_dim=core.head_dim, eps=core.eps, mscale=core.mscale)
+    core.cache.advance(length)
+    keys, values = core.cache.keys, core.cache.values
+    rows = core.cache.offset
+    return queries, keys[:, :, :rows], values[:, :, :rows]
+
+
+def prefill(core, raw_queries, raw_keys, raw_values, mask):
+    """The context [1, heads, T, D] of a prefill, or None, with nothing written, for a call
+    that `core` has to run."""
+    if not project_served(core, raw_queries, raw_keys, raw_values):
+        return None
+    if not 0 < core.scale < math.inf:
+        return None
+    length = raw_queries.shape[1]
+    if not mask_served(mask, length, core.cache.offset + length):
+        return None
+    sinks = core.sinks
+    if sinks is not None and (sinks.dtype != torch.bfloat16 or not sinks.is_contiguous()
+                              or sinks.numel() != core.heads):
+        return None
+    projected = project(core, raw_queries, raw_keys, raw_values)
+    if projected is None:
+        return None
+    queries, keys, values = projected
+    band = None
+    if mask is not None and not isinstance(mask, str):
+        band = mask.reshape(mask.shape[-2:])
+    out = ops.attention_prefill(queries, keys, values, scale=core.scale,
+                                causal=isinstance(mask, str) and mask == "causal", mask=band, sinks=sinks)
+    return out.unsqueeze(0)

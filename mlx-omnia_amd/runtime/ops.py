@@ -979,6 +979,126 @@ def attention_decode_noalloc(
     return out
 
 
+def _token_rows(t: torch.Tensor, width: int, name: str) -> tuple[int, int]:
+    """(tokens, row stride) of [..., T, width] bf16 rows with unit inner stride, 16-byte
+    vectors throughout; every leading axis has length 1."""
+    _require(t.dtype == BF16 and t.dim() >= 2 and t.shape[-1] == width and t.numel() == t.shape[-2] * width,
+             f"{name}: expected bf16 [T, {width}]")
+    stride = t.stride(-2) if t.shape[-2] > 1 else width
+    _require(t.stride(-1) == 1 and stride % 8 == 0 and stride >= width and t.data_ptr() % 16 == 0,
+             f"{name}: rows must be packed and 16-byte aligned")
+    return t.shape[-2], stride
+
+
+def _cache_rows(t: torch.Tensor, heads: int, rows: int, head_dim: int, name: str) -> int:
+    """Head stride of a [(1,) heads, rows, head_dim] bf16 view with packed rows."""
+    view = t[0] if t.dim() == 4 else t
+    _require(t.dtype == BF16 and tuple(view.shape) == (heads, rows, head_dim), f"{name}: shape {tuple(t.shape)}")
+    _require(view.stride(-1) == 1 and (rows <= 1 or view.stride(-2) == head_dim), f"{name}: rows must be packed")
+    stride = view.stride(0) if heads > 1 else rows * head_dim
+    _require(view.data_ptr() % 16 == 0 and stride % 8 == 0, f"{name}: must be 16-byte aligned")
+    return stride
+
+
+def attention_project(
+    raw_queries: torch.Tensor,
+    raw_keys: torch.Tensor,
+    raw_values: torch.Tensor,
+    query_weight: torch.Tensor | None,
+    key_weight: torch.Tensor | None,
+    angles: tuple[torch.Tensor, torch.Tensor] | None,
+    key_rows: torch.Tensor,
+    value_rows: torch.Tensor,
+    *,
+    heads: int,
+    kv_heads: int,
+    head_dim: int,
+    eps: float,
+    mscale: float = 1.0,
+    queries: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """The norms, the rotation and the cache write of an attention layer in one launch; see
+    `omnia_attention_project`. raw_queries [(1,) T, heads * D] and raw_keys, raw_values
+    [(1,) T, kv_heads * D] bf16 rows, weights [D] or None, angles the (cos, sin) rows
+    [T, pairs] fp32 or None, key_rows and value_rows [(1,) kv_heads, T, D] views of the
+    cache, written in place -> the queries [heads, T, D]."""
+    length, q_stride = _token_rows(raw_queries, heads * head_dim, "raw_queries")
+    k_length, k_stride = _token_rows(raw_keys, kv_heads * head_dim, "raw_keys")
+    v_length, v_stride = _token_rows(raw_values, kv_heads * head_dim, "raw_values")
+    _require(k_length == length and v_length == length, "attention_project: q, k, v differ in length")
+    tensors = [raw_queries, raw_keys, raw_values, key_rows, value_rows]
+    for weight, name in ((query_weight, "query_weight"), (key_weight, "key_weight")):
+        if weight is not None:
+            _dense(weight, BF16, name)
+            _require(weight.numel() == head_dim, f"{name}: must be [head_dim]")
+            tensors.append(weight)
+    pairs = table_stride = 0
+    if angles is not None:
+        cos, sin = angles
+        pairs = cos.shape[-1]
+        for rows, name in ((cos, "cos"), (sin, "sin")):
+            _require(rows.dtype == F32 and tuple(rows.shape) == (length, pairs) and rows.stride(-1) == 1,
+                     f"{name}: fp32 [T, pairs] with unit inner stride")
+            _require(rows.data_ptr() % 16 == 0, f"{name}: must be 16-byte aligned")
+        table_stride = cos.stride(0) if length > 1 else pairs
+        _require(length <= 1 or sin.stride(0) == table_stride, "attention_project: cos and sin row strides differ")
+        tensors += [cos, sin]
+    key_stride = _cache_rows(key_rows, kv_heads, length, head_dim, "key_rows")
+    value_stride = _cache_rows(value_rows, kv_heads, length, head_dim, "value_rows")
+    _require(on_rocm(*tensors), "attention_project: tensors must share one ROCm device")
+    queries = _out(queries, raw_queries, (heads, length, head_dim), BF16, "queries")
+    ptr = lambda t: t.data_ptr() if t is not None else None
+    call("omnia_attention_project", raw_queries.data_ptr(), q_stride, raw_keys.data_ptr(), k_stride,
+         raw_values.data_ptr(), v_stride, ptr(query_weight), ptr(key_weight),
+         cos.data_ptr() if angles is not None else None, sin.data_ptr() if angles is not None else None,
+         table_stride, pairs, float(mscale), float(eps), length, heads, kv_heads, head_dim,
+         queries.data_ptr(), key_rows.data_ptr(), key_stride, value_rows.data_ptr(), value_stride,
+         _stream(raw_queries))
+    return queries
+
+
+def attention_prefill(
+    queries: torch.Tensor,
+    keys: torch.Tensor,
+    values: torch.Tensor,
+    *,
+    scale: float,
+    causal: bool = False,
+    mask: torch.Tensor | None = None,
+    sinks: torch.Tensor | None = None,
+    out: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """Attention of a prompt's queries [heads, T, D] over the cached rows [(1,) kv_heads,
+    rows, D] (views with packed rows, this prompt's T rows the last); see
+    `omnia_attention_prefill`. mask: boolean [T, rows] (True attends) with unit inner
+    stride, or None; sinks [heads] bf16 or None -> [heads, T, D]."""
+    _dense(queries, BF16, "queries")
+    _require(queries.dim() == 3, "attention_prefill: queries must be [heads, T, D]")
+    heads, length, head_dim = queries.shape
+    kv_heads, rows = keys.shape[-3], keys.shape[-2]
+    key_stride = _cache_rows(keys, kv_heads, rows, head_dim, "keys")
+    value_stride = _cache_rows(values, kv_heads, rows, head_dim, "values")
+    tensors = [queries, keys, values]
+    mask_stride = 0
+    if mask is not None:
+        _require(mask.dtype == torch.bool and tuple(mask.shape) == (length, rows)
+                 and (rows <= 1 or mask.stride(-1) == 1), "attention_prefill: mask must be boolean [T, rows]")
+        mask_stride = mask.stride(0) if length > 1 else rows
+        _require(mask_stride >= rows, "attention_prefill: mask rows overlap")
+        tensors.append(mask)
+    if sinks is not None:
+        _require(sinks.dtype == BF16 and sinks.is_contiguous() and sinks.numel() == heads,
+                 "attention_prefill: sinks must be contiguous bf16 [heads]")
+        tensors.append(sinks)
+    _require(on_rocm(*tensors), "attention_prefill: tensors must share one ROCm device")
+    out = _out(out, queries, (heads, length, head_dim), BF16, "out")
+    call("omnia_attention_prefill", queries.data_ptr(), keys.data_ptr(), values.data_ptr(), key_stride,
+         value_stride, heads, kv_heads, head_dim, length, rows, int(causal),
+         mask.data_ptr() if mask is not None else None, mask_stride,
+         sinks.data_ptr() if sinks is not None else None, float(scale), out.data_ptr(), _stream(queries))
+    return out
+
+
 @dataclass(frozen=True)
 class Mxfp4Leaf:
     """An MXFP4 matrix set as the kernels read it: weight [..., rows, features / 8]

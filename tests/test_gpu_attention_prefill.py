@@ -1,0 +1,130 @@
+"""The prefill kernels (csrc/attention_prefill.hip) against the Core chain on the same device.
+
+Sizes straddle the kernel's tiles (32 queries a wave, 64 rows a tile), every way a
+workgroup's waves split into heads and queries, both head widths, causal, unmasked and
+boolean masks, with and without sinks, gains, rotation and earlier rows.
+
+Bar: the bf16 bar (assert_bf16_close), at least 98% of the context bit-identical to the
+fp32 Core chain (both round once from fp32 sums of the same products in another order: a
+value flips where the sums' difference, about sqrt(rows) 2^-24 of it, crosses a rounding
+point, so well under 1% do); the cache rows likewise at 99.9%, values bit-exact.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from mlx_omnia_amd.kernels.resolve import FALLBACKS
+from mlx_omnia_amd.kernels.attention import AttentionStep, FixedKVCache, KVCache
+from mlx_omnia_amd.kernels.qkv_rope import AngleAtlas, AngleTable
+from util import assert_bf16_close, bits_of
+
+pytestmark = pytest.mark.gpu
+
+
+class Layer:
+    """Two steps over equal caches: the binding's and the Core chain's."""
+
+    def __init__(self, seed, heads, kv_heads, d, past, tokens, *, sinks=False, gains=True, pairs=None,
+                 mscale=1.0, growing=None, angles=None):
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        self.normal = lambda *shape, s=1.0, m=0.0: (
+            m + s * torch.randn(shape, generator=gen, device="cuda")).to(torch.bfloat16)
+        pairs = d // 2 if pairs is None else pairs
+        sink = self.normal(heads, s=2.0) if sinks else None
+        declare = dict(heads=heads, kv_heads=kv_heads, head_dim=d, scale=d ** -0.5, dtype=torch.bfloat16,
+                       rotary_pairs=pairs, mscale=mscale, sinks=sink,
+                       angles=angles or AngleAtlas(pairs, base=1e4, rows=past + tokens + 8, device="cuda"))
+        if gains:
+            declare.update(query_weight=self.normal(d, s=0.1, m=1.0), key_weight=self.normal(d, s=0.1, m=1.0))
+        keys, values = self.normal(1, kv_heads, past, d), self.normal(1, kv_heads, past, d)
+        self.caches, self.steps = [], []
+        for reference in (False, True):
+            cache = KVCache() if sinks else FixedKVCache.empty(kv_heads, past + tokens + 3, d, device="cuda")
+            if past:
+                cache.update_and_fetch(keys, values)
+            self.caches.append(cache)
+            self.steps.append(AttentionStep(cache, reference=reference, **declare))
+        self.raw = [self.normal(1, tokens, n * d) for n in (heads, kv_heads, kv_heads)]
+        self.past, self.tokens = past, tokens
+
+    def check(self, mask, raw=None, fallbacks=0):
+        raw = raw or self.raw
+        before = sum(FALLBACKS.values())
+        got = self.steps[0](*raw, mask=mask)
+        assert sum(FALLBACKS.values()) == before + fallbacks
+        want = self.steps[1](*raw, mask=mask)
+        assert got.shape == want.shape and got.is_contiguous()
+        assert_bf16_close(bits_of(got), bits_of(want), min_exact=0.98)
+        ours, core = self.caches
+        assert ours.offset == core.offset == self.past + self.tokens
+        if isinstance(ours, FixedKVCache):
+            assert int(ours.position.item()) == ours.offset
+        assert ours.keys.shape == core.keys.shape
+        assert_bf16_close(bits_of(ours.keys), bits_of(core.keys), min_exact=0.999)
+        assert torch.equal(ours.values, core.values)
+        return got
+
+
+@pytest.mark.parametrize("tokens,past", [(2, 0), (31, 0), (32, 1), (33, 31), (64, 0), (65, 63), (129, 64),
+                                         (300, 77), (7, 1000)])
+@pytest.mark.parametrize("heads,kv_heads", [(2, 2), (4, 2), (8, 2), (8, 1)])
+def test_causal_prefill_matches_the_core_chain(tokens, past, heads, kv_heads):
+    print(f"prefill d=128 H={heads}/{kv_heads} T={tokens} past={past}", flush=True)
+    Layer(tokens + past, heads, kv_heads, 128, past, tokens).check("causal")
+
+
+@pytest.mark.parametrize("tokens,past", [(2, 0), (33, 100), (64, 64), (200, 0)])
+@pytest.mark.parametrize("mask", ["causal", "band", None])
+def test_sink_prefill_matches_the_core_chain(tokens, past, mask):
+    print(f"prefill sinks T={tokens} past={past} mask={mask}", flush=True)
+    layer = Layer(tokens + past + 1, 16, 2, 64, past, tokens, sinks=True, gains=False)
+    if mask == "band":
+        query = past + torch.arange(tokens, device="cuda")[:, None]
+        row = torch.arange(past + tokens, device="cuda")[None]
+        mask = ((row <= query) & (row > query - 40))[None, None]
+        mask[:, :, 0] = False     # the first query attends the sink alone: zeros
+    got = layer.check(mask)
+    if torch.is_tensor(mask):
+        assert not bool(got[0, :, 0].any())
+
+
+def test_partial_rotation_factor_and_strided_rows():
+    layer = Layer(5, 8, 2, 128, 20, 50, pairs=32, mscale=1.3465735912322998)
+    fused = layer.normal(1, 50, 12 * 128)   # q, k and v as slices of one projection's rows
+    layer.check("causal", raw=[fused[..., :1024], fused[..., 1024:1280], fused[..., 1280:]])
+    table = AngleTable(*(torch.rand(64, 64, device="cuda") for _ in range(2)))
+    Layer(6, 4, 4, 128, 3, 40, angles=table).check(None)
+
+
+def test_calls_the_kernels_do_not_compute_stay_with_the_core_chain():
+    layer = Layer(7, 4, 2, 128, 10, 40)
+    additive = torch.zeros((40, 50), device="cuda")
+    layer.check(additive, fallbacks=1)
+    layer = Layer(8, 4, 2, 128, 10, 40)
+    raw = [layer.raw[0].clone().requires_grad_(), *layer.raw[1:]]
+    step = layer.steps[0]
+    out = step(*raw, mask="causal")
+    assert out.requires_grad
+    short = AngleTable(*(torch.rand(20, 64, device="cuda") for _ in range(2)))
+    with pytest.raises(RuntimeError):      # the table ends before the prompt does
+        Layer(9, 4, 2, 128, 0, 40, angles=short).steps[0](*layer.raw, mask="causal")
+    cache = layer.caches[1]
+    with pytest.raises(ValueError):
+        layer.steps[0](*layer.raw, mask="causal")   # the cache is full
+    assert cache.offset == 10
+
+
+def test_a_row_that_attends_nothing_is_nan_and_later_rows_are_not_read():
+    layer = Layer(10, 4, 2, 128, 0, 70)
+    mask = torch.ones((70, 70), dtype=torch.bool, device="cuda").tril()
+    mask[66] = False
+    got, want = (step(*layer.raw, mask=mask) for step in layer.steps)
+    assert torch.equal(got.isnan(), want.isnan()) and bool(got[0, :, 66].isnan().all())
+    keep = ~want.isnan()
+    assert_bf16_close(bits_of(got[keep]), bits_of(want[keep]), min_exact=0.98)
+    cache = layer.caches[0]
+    cache.keys[:, :, 70:], cache.values[:, :, 70:] = float("nan"), float("inf")
+    cache.offset = 0
+    again = layer.steps[0](*layer.raw, mask=mask)
+    assert np.array_equal(bits_of(got), bits_of(again))
