@@ -449,6 +449,23 @@ int32_t omnia_moe_down_combine_nvfp4_shared(const uint16_t* act, const uint32_t*
                                             const float* weights, int64_t tokens, int64_t top_k,
                                             const uint16_t* residual, uint16_t* out, hipStream_t stream);
 
+/* Workspace bytes of omnia_moe_down_combine_nvfp4_shared_grouped: 0 where the per-token
+ * entry above serves the call better (few tokens, or a contraction other than 512).
+ * -EINVAL for a bad geometry. Pure; touches no device. */
+int64_t omnia_moe_nvfp4_shared_workspace_bytes(int64_t experts, int64_t hidden, int64_t inner,
+                                               int64_t tokens, int64_t top_k);
+
+/* omnia_moe_down_combine_nvfp4_shared over a prompt: the same arguments and results (the
+ * fp32 sums in another order) with the tokens grouped by expert, in a caller's workspace of
+ * at least omnia_moe_nvfp4_shared_workspace_bytes bytes, 16-byte aligned. Where that is 0
+ * the call is the per-token entry's. */
+int32_t omnia_moe_down_combine_nvfp4_shared_grouped(
+    const uint16_t* act, const uint32_t* weight, const uint8_t* scales, int64_t experts,
+    const uint32_t* shared_weight, const uint8_t* shared_scales, int64_t hidden, int64_t inner,
+    const int32_t* chosen, const float* weights, int64_t tokens, int64_t top_k,
+    const uint16_t* residual, void* workspace, int64_t workspace_bytes, uint16_t* out,
+    hipStream_t stream);
+
 /* Dense SwiGLU MLP of one token, first half: the fused gate||up projection with the
  * SwiGLU applied in bf16 steps,
  *   g = bf16(sum_h x[h] * fused[n, h]),  u = bf16(sum_h x[h] * fused[inner + n, h])   fp32 sums

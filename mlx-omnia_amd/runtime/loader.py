@@ -78,6 +78,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                            _P, _P]),
     "omnia_moe_down_combine_nvfp4_shared": (_I32, [_P, _P, _P, _I64, _P, _P, _I64, _I64, _P, _P, _I64, _I64, _P,
                                                    _P, _P]),
+    "omnia_moe_nvfp4_shared_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64]),
+    "omnia_moe_down_combine_nvfp4_shared_grouped": (_I32, [_P, _P, _P, _I64, _P, _P, _I64, _I64, _P, _P, _I64, _I64,
+                                                           _P, _P, _I64, _P, _P]),
     "omnia_moe_gate_up_nvfp4_ordinal": (_I32, [_P, _P, _P, _I64, _I64, _I64, _P, _I64, _P, _P]),
     "omnia_dense_gate_up_swiglu": (_I32, [_P, _P, _I64, _I64, _P, _P]),
     "omnia_dense_down_residual": (_I32, [_P, _P, _P, _I64, _I64, _P, _P]),

@@ -1348,6 +1348,14 @@ def moe_down_combine_nvfp4_shared(
     _require(on_rocm(act, chosen, weights, residual, *leaf.tensors(), *shared.tensors()),
              f"{name}: tensors must share one ROCm device")
     out = _out(out, act, (tokens, hidden), BF16, "out")
+    nbytes = library().omnia_moe_nvfp4_shared_workspace_bytes(experts, hidden, inner, tokens, top_k)
+    if nbytes > 0:   # a prompt: the tokens grouped by expert, on the matrix cores
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=act.device)
+        call("omnia_moe_down_combine_nvfp4_shared_grouped", act.data_ptr(), leaf.weight.data_ptr(),
+             leaf.scales.data_ptr(), experts, shared.weight.data_ptr(), shared.scales.data_ptr(), hidden, inner,
+             chosen.data_ptr(), weights.data_ptr(), tokens, top_k, residual.data_ptr(), workspace.data_ptr(),
+             nbytes, out.data_ptr(), _stream(act))
+        return out
     call("omnia_moe_down_combine_nvfp4_shared", act.data_ptr(), leaf.weight.data_ptr(), leaf.scales.data_ptr(),
          experts, shared.weight.data_ptr(), shared.scales.data_ptr(), hidden, inner, chosen.data_ptr(),
          weights.data_ptr(), tokens, top_k, residual.data_ptr(), out.data_ptr(), _stream(act))

@@ -20,7 +20,7 @@ import torch
 
 from mlx_omnia_amd.runtime import ops
 from oracle import nvfp4
-from oracle.bf16 import from_float
+from oracle.bf16 import from_float, to_f32
 from util import assert_bf16_close, bits_of, to_device
 
 pytestmark = pytest.mark.gpu
@@ -44,7 +44,7 @@ def _leaf(stack):
                          torch.from_numpy(stack.scales).cuda(), None)
 
 
-def _run(seed, tokens, top_k, hidden, inner, experts, *, special=False, invalid=False):
+def _case(seed, tokens, top_k, hidden, inner, experts, *, special=False, invalid=False):
     rng = np.random.default_rng(seed)
     routed = _stack(rng, experts, hidden, inner, special=special)
     shared = _stack(rng, 1, hidden, inner, special=special)
@@ -55,12 +55,21 @@ def _run(seed, tokens, top_k, hidden, inner, experts, *, special=False, invalid=
         chosen[-1, -1] = experts
     weights = rng.dirichlet(np.ones(max(top_k, 1)), size=tokens)[:, :top_k].astype(np.float32)
     residual = from_float(rng.standard_normal((tokens, hidden)))
+    return routed, shared, act, chosen, weights, residual
+
+
+def _both(case):
+    routed, shared, act, chosen, weights, residual = case
     got = ops.moe_down_combine_nvfp4_shared(
         to_device(act), _leaf(routed), _leaf(nvfp4.Stack(shared.weight[0], shared.scales[0])),
         torch.from_numpy(chosen).cuda(), torch.from_numpy(weights).cuda(), to_device(residual))
     want = nvfp4.down_combine_shared(act, routed, nvfp4.Stack(shared.weight[0], shared.scales[0]),
                                      chosen, weights, residual)
     return bits_of(got), want
+
+
+def _run(*args, **options):
+    return _both(_case(*args, **options))
 
 
 @pytest.mark.parametrize("tokens,top_k,hidden,inner,experts", [
@@ -163,3 +172,34 @@ def test_golden_fixture():
         to_device(golden["act"]), leaf("down"), leaf("shared"), torch.from_numpy(golden["chosen"]).cuda(),
         torch.from_numpy(golden["weights"]).cuda(), to_device(golden["residual"]))
     assert_bf16_close(bits_of(out), golden["out"], min_exact=0.99)
+
+
+@pytest.mark.parametrize("tokens,top_k,hidden,experts", [
+    (24, 10, 2048, 512),    # about the fewest tokens grouped by expert; most experts idle
+    (300, 4, 100, 60),      # 64 tokens a tile; a short last row tile, 4-byte rows of out
+    (1200, 1, 65, 2),       # odd rows: the scalar epilogue
+    (100, 31, 72, 400),     # the most routed slots, 16 tokens a tile
+    (1500, 2, 64, 600),     # experts without a pair
+    (150, 8, 1408, 500),    # two row tiles a workgroup, the second past the last row
+])
+def test_grouped_prompt_matches_oracle(tokens, top_k, hidden, experts):
+    """Each d is one fp32 sum of 512 exact products rounded to bf16, in another order than the
+    per-token kernel's, so some flip to the neighbouring bf16: at least 99% of the outputs are
+    bit-identical to the oracle's. A flip of d_s, of a weighted term or of a running total moves
+    the output by at most one ulp of it, 2^-7 S with S = sum |w_s d_s| + |d_shared| + |residual|
+    (every running total is at most S); the bound is three of them in one output."""
+    print(f"moe_down_combine_nvfp4_shared grouped tokens={tokens} top_k={top_k} hidden={hidden}", flush=True)
+    assert ops.library().omnia_moe_nvfp4_shared_workspace_bytes(experts, hidden, 512, tokens, top_k) > 0
+    case = _case(tokens + top_k, tokens, top_k, hidden, 512, experts, special=tokens == 300, invalid=tokens == 100)
+    routed, shared, act, chosen, weights, residual = case
+    got, want = _both(case)
+    assert float(np.mean(got == want)) >= 0.99
+    size = np.abs(to_f32(residual).astype(np.float64))
+    x = to_f32(act).astype(np.float64)
+    size += np.abs(x[:, top_k] @ nvfp4.dequantize(shared)[0].T)
+    for e in range(experts):
+        token, slot = np.nonzero(chosen == e)
+        if token.size:
+            d = np.abs(x[token, slot] @ nvfp4.dequantize(nvfp4.Stack(routed.weight[e:e + 1], routed.scales[e:e + 1]))[0].T)
+            np.add.at(size, token, d * weights[token, slot][:, None])
+    assert np.all(np.abs(to_f32(got) - to_f32(want)) <= 3 * 2.0 ** -7 * size)
