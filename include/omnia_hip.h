@@ -228,10 +228,12 @@ int32_t omnia_pack_router_weight(const uint16_t* router_weight, int64_t experts,
  * x, branch [rows, hidden] bf16; norm_weight [hidden] bf16; packed_router: the router
  * weight [experts, hidden] bf16 as omnia_pack_router_weight wrote it.
  * hidden in {2048, 4096}, experts in {128, 256}; k <= 64.
- * With rows <= 512 and `logits` given (decode steps and short prefills) the launch is
- * two dispatches: the projection spread over many workgroups, every logit an fp64 dot
- * product rounded once, then the selection of omnia_softmax_topk over the written
- * logits. The outputs are the same bits either way.
+ * With `logits` given the projection is a dispatch of its own, spread over the chip: for
+ * rows * experts <= 32768 (decode steps) every logit an fp64 dot product rounded once, for
+ * more rows a matrix-core product with the logits its error bound leaves open recomputed
+ * (hidden 2048 with 128 experts: up to 1280 rows, then the fused dispatch); then the
+ * selection of omnia_softmax_topk over the written logits. The outputs are the same bits
+ * either way.
  * Replaces: core/kernels/route/residual.py:117-299 (`residual_rms_router`, the
  * one-token residual join with the router gemv fused), generalised to many tokens and
  * to softmax routing; the Core chain is add_norm/default.py:28-29 followed by
@@ -267,9 +269,9 @@ int32_t omnia_sigmoid_topk(const void* logits, int64_t stride, int32_t logits_fp
  *   logits [rows, experts] bf16 or null; keys [rows, experts] uint32 or null;
  *   indices [rows, k] int32 and weights [rows, k] fp32, both or neither.
  * Every logit is the correctly rounded bf16 of the exact dot product, so the keys and
- * the selection equal those computed from the exact logits. With rows <= 512 and `logits`
- * given the launch is the two dispatches of omnia_residual_rms_router's decode path,
- * the second omnia_sigmoid_topk over the written logits.
+ * the selection equal those computed from the exact logits. With `logits` given the launch
+ * is the dispatches of omnia_residual_rms_router with its logits given, the last one
+ * omnia_sigmoid_topk over the written logits.
  * Replaces: core/kernels/route/residual.py:117-299 (`residual_rms_router` with its
  * `correction_bias`, emitting logits and ordinal keys; its T = 1 only).
  * hidden 2048 or 4096, experts 128 or 256. */

@@ -90,9 +90,8 @@ class HipResidualRouter(ResidualRouterStrategy):
                    routing)
 
     def __call__(self, x, projected):
-        # Up to 64 tokens (decode steps, short prefills) take the library's decode path,
-        # which needs the logits written out; more tokens run the one fused dispatch
-        # without them.
+        # Few tokens (decode steps, short prefills) take the library's decode path, which
+        # needs the logits written out; more tokens run the one fused dispatch without them.
         decode = x.numel() // x.shape[-1] <= ops.ROUTER_SELECT_VIA_DECODE_ROWS
         if self.routing.bias is not None:
             summed, normalized, _, _, indices, weights = ops.residual_rms_router_sigmoid(

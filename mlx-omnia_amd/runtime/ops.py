@@ -408,14 +408,12 @@ def pack_router_weight(router_weight: torch.Tensor) -> PackedRouterWeight:
     return PackedRouterWeight(buffer, int(experts), int(hidden))
 
 
-# At most this many rows with the logits written out take the fused router's decode
-# path: every logit an fp64 dot product spread over the chip, then the selection kernel
-# (two dispatches); more rows run the fused dispatch.
-ROUTER_DECODE_ROWS = 512
-# A selection-only call up to this many rows is faster on the decode path (its logits
-# then written to a scratch tensor) than in the fused dispatch: measured on MI355X at
-# 2048 x 128, 9.9 against 13.0 us at 17 rows, 11.0 against 13.6 at 64, even at 128.
-ROUTER_SELECT_VIA_DECODE_ROWS = 64
+# A selection-only call up to this many rows is faster with its logits written to a scratch
+# tensor (the library's decode path, or its product path at 256 experts of hidden 4096) than
+# in the fused dispatch: measured on MI355X, 12.3 against 15.1 us at 96 rows of 2048 x 128,
+# 19.7 against 19.8 at 128 of 2048 x 256, 20.4 against 25.2 at 128 of 4096 x 128, even or
+# slower above.
+ROUTER_SELECT_VIA_DECODE_ROWS = 128
 
 
 def residual_rms_router(
@@ -437,8 +435,8 @@ def residual_rms_router(
     `omnia_residual_rms_router`. `router` is a packed weight (`pack_router_weight`, what a
     strategy holds) or the [experts, hidden] bf16 weight itself, then packed for this call.
     Returns (summed, normalized, logits or None, indices, weights). Writing the logits
-    makes every logit exact: the decode path up to 512 rows, above it the fused dispatch
-    with every unsure logit recomputed in fp64 (slower than selecting alone)."""
+    makes every logit exact, which costs more than selecting alone from a few hundred rows
+    on."""
     hidden = norm_weight.numel()
     if not isinstance(router, PackedRouterWeight):
         _require(router.dim() == 2 and router.shape[-1] == hidden,
@@ -523,9 +521,9 @@ def residual_rms_router_sigmoid(
     weights or None); an output passed in is written in place.
 
     Writing the logits or the keys (the defaults: the reference's own outputs) makes
-    every logit exact. Up to 512 rows that is the decode path (about 10 us at 17 rows,
-    32 us at 512, at 2048 x 128); above it the fused dispatch recomputes every unsure
-    logit in fp64, about 2.6 times the selection-only launch at [4096, 2048] x 128. A
+    every logit exact: about 10 us at 17 rows of 2048 x 128, 25 us at 512, about twice the
+    selection-only launch at [4096, 2048] x 128. Keys without logits run the fused dispatch
+    at any row count, so ask for both. A
     caller that only needs the selection passes emit_logits=False, emit_keys=False."""
     hidden = norm_weight.numel()
     if not isinstance(router, PackedRouterWeight):
