@@ -53,10 +53,11 @@ class FixedKVCache:
         self.offset += rows
         self.position += rows
 
-    def claim(self, length: int, kv_heads: int, head_dim: int, like: torch.Tensor):
-        """The next `length` rows of both buffers, for a writer that then calls `advance`."""
-        rows = slice(self.offset, self.offset + length)
-        return self.keys[:, :, rows], self.values[:, :, rows]
+    def claim(self, length: int, kv_heads: int, head_dim: int, like: torch.Tensor) -> None:
+        """Make sure of the next `length` rows, for a writer that puts them into the buffers
+        itself and then calls `advance`."""
+        if self.offset + length > self.capacity:
+            raise ValueError(f"cache of {self.capacity} rows cannot take row {self.offset + length - 1}")
 
     def update_and_fetch(self, keys: torch.Tensor, values: torch.Tensor):
         """Append [1, kv_heads, T, D] rows at the position; the rows written so far."""
@@ -133,15 +134,15 @@ class KVCache:
             grown[:, :, : buffer.shape[2]] = buffer
         return grown
 
-    def claim(self, length: int, kv_heads: int, head_dim: int, like: torch.Tensor):
-        """The next `length` rows of both buffers (grown to hold them), for a writer that
-        then calls `advance`."""
+    def claim(self, length: int, kv_heads: int, head_dim: int, like: torch.Tensor) -> None:
+        """Make sure of the next `length` rows of both buffers (grown to hold them, as
+        `update_and_fetch` grows them), for a writer that puts them there itself and then
+        calls `advance`."""
         needed = self.offset + length
         if self.capacity < needed or self.values.shape[2] < needed:
             row = like.new_empty((1, kv_heads, 0, head_dim))
             self.keys = self._reserve(self.keys, needed, row)
             self.values = self._reserve(self.values, needed, row)
-        return self.keys[:, :, self.offset : needed], self.values[:, :, self.offset : needed]
 
     def advance(self, rows: int = 1) -> None:
         """Account for rows a writer put into the buffers itself."""

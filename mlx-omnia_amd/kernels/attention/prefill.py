@@ -15,6 +15,7 @@ from __future__ import annotations
 import math
 
 import torch
+from torch.autograd import forward_ad
 from torch.overrides import _get_current_function_mode_stack
 from torch.utils._device import DeviceContext
 
@@ -25,28 +26,24 @@ from ..qkv_rope.kernel import AngleTable
 from .cache import FixedKVCache, KVCache
 
 HEAD_DIMS = (64, 128)
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def plain_call(*tensors: torch.Tensor) -> bool:
     """Ordinary tensors on the current ROCm device, with nothing following the operations
     on them: a kernel may then stand in for torch ops."""
-    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0:
+    if torch._C._len_torch_dispatch_stack() or torch.compiler.is_compiling():
         return False
-    if torch._C._functorch.peek_interpreter_stack() is not None:
+    if torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0:
         return False
-    if any(type(mode) is not DeviceContext for mode in _get_current_function_mode_stack()):
+    if torch._C._len_torch_function_stack() and any(
+            type(mode) is not DeviceContext for mode in _get_current_function_mode_stack()):
         return False
-    if torch.autograd.forward_ad._current_level >= 0:
-        return False
-    if any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in tensors):
-        return False
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
-        return False
-    return hip_device(*tensors) and tensors[0].device.index == torch.cuda.current_device()
-
-
-def _rows_readable(raw: torch.Tensor, length: int, width: int) -> bool:
-    return raw.dtype == torch.bfloat16 and tuple(raw.shape) == (1, length, width)
+    followed = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in _PLAIN or (followed and t.requires_grad):
+            return False
+    return hip_device(*tensors) and tensors[0].get_device() == torch._C._cuda_getDevice()
 
 
 def _gain_readable(weight: torch.Tensor | None, head_dim: int) -> bool:
@@ -75,12 +72,15 @@ def _cache_writable(cache, length: int, kv_heads: int, head_dim: int) -> bool:
 def project_served(core, raw_queries, raw_keys, raw_values) -> bool:
     """Whether `project` computes this call's prologue as `core` (a `DefaultAttentionStep`)
     does."""
-    if raw_queries.dim() != 3 or core.head_dim not in HEAD_DIMS or core.heads % core.kv_heads:
+    d = core.head_dim
+    if raw_queries.dim() != 3 or d not in HEAD_DIMS or core.heads % core.kv_heads:
         return False
-    length, d = raw_queries.shape[1], core.head_dim
-    if length == 0 or not (_rows_readable(raw_queries, length, core.heads * d)
-                           and _rows_readable(raw_keys, length, core.kv_heads * d)
-                           and _rows_readable(raw_values, length, core.kv_heads * d)):
+    length = raw_queries.shape[1]
+    rows = (1, length, core.kv_heads * d)
+    if (length == 0 or raw_queries.shape != (1, length, core.heads * d) or raw_keys.shape != rows
+            or raw_values.shape != rows):
+        return False
+    if not raw_queries.dtype == raw_keys.dtype == raw_values.dtype == torch.bfloat16:
         return False
     if core.rotary_pairs % 8 or 2 * core.rotary_pairs > d:
         return False
@@ -89,8 +89,7 @@ def project_served(core, raw_queries, raw_keys, raw_values) -> bool:
     cache = core.cache
     if not _cache_writable(cache, length, core.kv_heads, d):
         return False
-    held = [t for t in (core.query_weight, core.key_weight, core.sinks, getattr(cache, "keys", None),
-                        getattr(cache, "values", None)) if t is not None]
+    held = [t for t in (core.query_weight, core.key_weight, core.sinks, cache.keys, cache.values) if t is not None]
     return plain_call(raw_queries, raw_keys, raw_values, *held)
 
 
@@ -105,11 +104,12 @@ def mask_served(mask, length: int, rows: int) -> bool:
 
 
 def _readable_rows(raw: torch.Tensor) -> torch.Tensor:
-    """The [T, width] rows, copied where the kernel could not read them in place."""
-    rows = raw[0]
-    if rows.stride(-1) != 1 or rows.stride(0) % 8 or rows.stride(0) < rows.shape[1] or rows.data_ptr() % 16:
-        rows = rows.clone(memory_format=torch.contiguous_format)
-    return rows
+    """The rows [1, T, width], copied where the kernel could not read them in place."""
+    stride = raw.stride(1)
+    if (raw.stride(2) != 1 or (raw.shape[1] > 1 and (stride % 8 or stride < raw.shape[2]))
+            or raw.data_ptr() % 16):
+        raw = raw.clone(memory_format=torch.contiguous_format)
+    return raw
 
 
 def _angle_rows(core, length: int, device):
@@ -123,11 +123,13 @@ def _angle_rows(core, length: int, device):
         cos, sin = rows[:, :pairs], rows[:, pairs : 2 * pairs]
     else:
         cos, sin = core._angles(offset, length, device)
+    shape = (length, pairs)
     for rows in (cos, sin):
-        if (rows.dtype != torch.float32 or rows.device != device or tuple(rows.shape) != (length, pairs)
-                or rows.stride(-1) != 1 or rows.data_ptr() % 16 or (length > 1 and rows.stride(0) % 4)
-                or rows.stride(0) != cos.stride(0)):
+        if (rows.dtype != torch.float32 or rows.device != device or rows.shape != shape
+                or rows.stride(-1) != 1 or rows.data_ptr() % 16):
             return None
+    if length > 1 and (cos.stride(0) % 4 or sin.stride(0) != cos.stride(0)):
+        return None
     return cos, sin
 
 
@@ -140,15 +142,15 @@ def project(core, raw_queries, raw_keys, raw_values):
         angles = _angle_rows(core, length, device)
         if angles is None:
             return None
-    key_rows, value_rows = core.cache.claim(length, core.kv_heads, core.head_dim, raw_keys)
+    cache = core.cache
+    cache.claim(length, core.kv_heads, core.head_dim, raw_keys)
     queries = ops.attention_project(
         _readable_rows(raw_queries), _readable_rows(raw_keys), _readable_rows(raw_values),
-        core.query_weight, core.key_weight, angles, key_rows, value_rows, heads=core.heads,
-        kv_heads=core.kv_heads, head_dim=core.head_dim, eps=core.eps, mscale=core.mscale)
-    core.cache.advance(length)
-    keys, values = core.cache.keys, core.cache.values
-    rows = core.cache.offset
-    return queries, keys[:, :, :rows], values[:, :, :rows]
+        core.query_weight, core.key_weight, angles, cache.keys, cache.values, cache.offset,
+        heads=core.heads, kv_heads=core.kv_heads, head_dim=core.head_dim, eps=core.eps, mscale=core.mscale)
+    cache.advance(length)
+    rows = cache.offset
+    return queries, cache.keys[:, :, :rows], cache.values[:, :, :rows]
 
 
 def prefill(core, raw_queries, raw_keys, raw_values, mask):

@@ -81,6 +81,7 @@ class AngleAtlas:
         # fp64: the frequencies f_i; fp32: the inverse row base ** (2i / D).
         self.frequencies = torch.from_numpy(np.ascontiguousarray(frequencies)).to(self.device)
         self.atlas = torch.empty((0, 2 * pairs), dtype=torch.float32, device=self.device)
+        self._viewed = self._table = None
         self.grow(rows)
 
     @property
@@ -125,7 +126,11 @@ class AngleAtlas:
             self.grow(max(2 * self.rows, position + 1))
 
     def table(self) -> AngleTable:
-        return AngleTable.from_atlas(self.atlas)
+        """The atlas as it stands, viewed as cosines and sines (the views made once for each
+        growth)."""
+        if self._viewed is not self.atlas:
+            self._table, self._viewed = AngleTable.from_atlas(self.atlas), self.atlas
+        return self._table
 
     def __call__(self, offset: int, length: int) -> torch.Tensor:
         """Rows offset .. offset+length-1, cosines then sines (the `Angles` contract)."""

@@ -100,8 +100,9 @@ class HipQkNormRope(QkvRopeStrategy):
         if rows.stride(-1) != 1:
             rows = rows.contiguous()
         q_width, kv_width = self.heads * self.head_dim, self.kv_heads * self.head_dim
-        raw_q = rows[:, :q_width].unflatten(-1, (self.heads, self.head_dim))
-        raw_k = rows[:, q_width : q_width + kv_width].unflatten(-1, (self.kv_heads, self.head_dim))
+        length = rows.shape[0]
+        raw_q = rows[:, :q_width].view(length, self.heads, self.head_dim)
+        raw_k = rows[:, q_width : q_width + kv_width].view(length, self.kv_heads, self.head_dim)
         cos, sin, table_offset = self._tables(offset, rows.shape[0])
         q, k = ops.qk_norm_rope(
             raw_q, raw_k, self.q_norm, self.k_norm, cos, sin, offset=table_offset,

@@ -158,7 +158,7 @@ def last_error() -> str:
 
 def call(name: str, *args: object) -> None:
     """Invoke one entry point and turn a non-zero return code into an exception."""
-    rc = getattr(library(), name)(*args)
+    rc = getattr(_library or library(), name)(*args)
     if rc == 0:
         return
     message = f"{name}: {last_error()} (code {rc})"
