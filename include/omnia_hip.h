@@ -602,6 +602,12 @@ int32_t omnia_attention_project(const uint16_t* raw_queries, int64_t query_strid
                                 uint16_t* queries, uint16_t* key_rows, int64_t key_head_stride,
                                 uint16_t* value_rows, int64_t value_head_stride, hipStream_t stream);
 
+/* Workspace bytes omnia_attention_prefill needs: the states of queries whose keys are walked
+ * by several workgroups (short prompts over many rows); 0 where one does. -EINVAL for a bad
+ * geometry. Pure; touches no device. */
+int64_t omnia_attention_prefill_workspace_bytes(int64_t heads, int64_t kv_heads, int64_t head_dim,
+                                                int64_t length, int64_t rows);
+
 /* Attention of `length` queries per head over `rows` cached rows (the queries are the last
  * `length` of them):
  *   s[h, t, r] = scale * (q[h, t] . keys[h / gqa, r]) where r is attended
@@ -610,7 +616,8 @@ int32_t omnia_attention_project(const uint16_t* raw_queries, int64_t query_strid
  * causal = 1: query t attends rows <= rows - length + t; a mask ([length, rows] bytes, rows
  * `mask_stride` apart, non-zero attends) is applied as well. A query that attends nothing
  * gives 0 / 0 (0 with a sink). queries, out [heads, length, D]; keys, values: head h, row r
- * at h * head_stride + r * D.
+ * at h * head_stride + r * D. workspace: at least omnia_attention_prefill_workspace_bytes,
+ * 16-byte aligned (null where that is 0).
  * Replaces: core/kernels/attention/default.py:132-156 (the attention of the Core chain at
  * T > 1, which a prefill runs).
  * head_dim 64 or 128; heads a multiple of kv_heads; scale positive and finite. */
@@ -619,7 +626,8 @@ int32_t omnia_attention_prefill(const uint16_t* queries, const uint16_t* keys,
                                 int64_t value_head_stride, int64_t heads, int64_t kv_heads,
                                 int64_t head_dim, int64_t length, int64_t rows, int32_t causal,
                                 const uint8_t* mask, int64_t mask_stride, const uint16_t* sinks,
-                                float scale, uint16_t* out, hipStream_t stream);
+                                float scale, void* workspace, int64_t workspace_bytes,
+                                uint16_t* out, hipStream_t stream);
 
 /* Calibration copy: dst[0 .. bytes) = src[0 .. bytes), 16-byte nontemporal loads and
  * stores, `vectors_per_thread` (1, 2 or 4) vectors per thread issued before the first

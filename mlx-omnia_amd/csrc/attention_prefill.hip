@@ -99,11 +99,22 @@ struct PrefillArgs {
   int64_t mask_stride;
   const uint16_t* sinks;    // [heads] or null
   uint16_t* out;            // [heads, length, D]
-  int heads, group, share, length, rows, causal;
+  float* partial;           // splits > 1: [splits, heads, length, D] unnormalised contexts, then
+                            // [splits, heads, length, 2] running maxima and sums
+  int heads, group, share, length, rows, causal, splits;
   float scale_log2, sink_log2;
 };
 
 constexpr int kWaveQueries = 32, kTileKeys = 64, kWaves = 4;
+constexpr int kTargetBlocks = 256, kMinSplitTiles = 4, kMaxSplits = 16;
+constexpr int kWindow = 64;   // tiles whose masks are looked through at a time
+
+// 4 mask bytes of any alignment (global memory reads need none on this target).
+__device__ __forceinline__ uint32_t mask_word(const uint8_t* at) {
+  uint32_t word;
+  __builtin_memcpy(&word, at, 4);
+  return word;
+}
 
 // A workgroup's four waves take 32 queries each: `share` heads of one kv head (the largest
 // of 1, 2, 4 dividing the group, so that the waves read the same keys), 4 / share runs of
@@ -121,15 +132,16 @@ constexpr int kWaveQueries = 32, kTileKeys = 64, kWaves = 4;
 //
 // Bound by the matrix cores and the softmax's VALU work about equally. The torch chain it
 // replaces wrote and read the fp32 scores five times and widened and repeated K and V:
-// 4,096 tokens, 32 heads over 4, D = 128, causal: 6,181 -> 314 us (438 TFLOP/s of the
+// 4,096 tokens, 32 heads over 4, D = 128, causal: 6,181 -> 304 us a call (460 TFLOP/s of the
 // products counted once, twice that on the matrix cores); 777 tokens after 1,500, 64 heads
 // over 8, D = 64, sinks: 1,962 -> 81 us.
-template <int D>
+template <int D, bool kMasked>
 __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a) {
   constexpr int kSteps = D / 16, kBlocks = D / 32, kChunks = D / 8;
   constexpr int kLoads = kTileKeys * kChunks / 256;   // 16-byte vectors a thread stages, each of K and V
   constexpr int kTile = kTileKeys * D;                // elements of one tile
   __shared__ __attribute__((aligned(16))) uint16_t lds[4 * kTile];   // K, V of two stages
+  __shared__ unsigned long long window_flags[kMasked ? 2 : 1];
 
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int column = lane % 32, half = lane / 32;
@@ -148,7 +160,12 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
   const int past = a.rows - a.length;
   const int last_query = min((query_tile + 1) * tile_queries, a.length) - 1;
   const int row_end = a.causal ? past + last_query + 1 : a.rows;
-  const int tiles = (row_end + kTileKeys - 1) / kTileKeys;
+  // This workgroup's share of the attended tiles.
+  const int split = blockIdx.y;
+  const int all_tiles = (row_end + kTileKeys - 1) / kTileKeys;
+  const int split_tiles = (all_tiles + a.splits - 1) / a.splits;
+  const int first_tile = split * split_tiles;
+  const int tiles = min(first_tile + split_tiles, all_tiles);   // past the last
   const uint16_t* keys = a.keys + kv_head * a.key_stride;
   const uint16_t* values = a.values + kv_head * a.value_stride;
 
@@ -204,32 +221,89 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
   f32x16 out[kBlocks];
 #pragma unroll
   for (int b = 0; b < kBlocks; ++b) out[b] = f32x16{};
-  float top = a.sinks != nullptr ? bf16_to_f32(a.sinks[head]) * a.sink_log2 : -INFINITY;
-  float total = a.sinks != nullptr && half == 0 ? 1.0f : 0.0f;
+  const bool sink = a.sinks != nullptr && split == 0;
+  float top = sink ? bf16_to_f32(a.sinks[head]) * a.sink_log2 : -INFINITY;
+  float total = sink && half == 0 ? 1.0f : 0.0f;
 
-  if (tiles > 0) {
-    load_tile(0);
+  // With a mask, the tiles in which any of the workgroup's queries attends anything: the
+  // masks of 64 tiles at a time are read 256 keys a load, so that the tiles outside a band
+  // cost their mask bytes and no more (2,000 tokens, 64 heads over 8, D = 64, a band of 128:
+  // 434 -> 86 us; 777 after 1,500: 217 -> 42).
+  uint64_t flags = ~uint64_t{0};
+  int window = -1;
+  auto look = [&](int w) {   // uniform over the workgroup, barriers inside
+    if (threadIdx.x == 0) window_flags[w & 1] = 0;
+    lds_barrier();
+    uint64_t found = 0;
+    const int queries = min(tile_queries, a.length - query_tile * tile_queries);
+    const int end = min(tiles, (w + 1) * kWindow) * kTileKeys;
+    for (int r = wave; r < queries; r += kWaves) {
+      const uint8_t* row = a.mask + static_cast<int64_t>(query_tile * tile_queries + r) * a.mask_stride;
+#pragma unroll 4
+      for (int key0 = w * kWindow * kTileKeys; key0 < end; key0 += 4 * kWave) {
+        const int key = key0 + 4 * lane;
+        uint32_t word = 0;
+        if (key + 4 <= a.rows) {
+          word = mask_word(row + key);
+        } else {
+          for (int i = key; i < a.rows; ++i) word |= row[i];
+        }
+        const uint64_t lanes = __ballot(word != 0);
+        const int at = key0 / kTileKeys - w * kWindow;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) found |= ((lanes >> (16 * i)) & 0xFFFF) != 0 ? uint64_t{1} << (at + i) : 0;
+      }
+    }
+    if (lane == 0 && found != 0) atomicOr(&window_flags[w & 1], static_cast<unsigned long long>(found));
+    lds_barrier();
+    flags = window_flags[w & 1];
+    window = w;
+  };
+  auto next_tile = [&](int tile) {   // the first tile from `tile` on to walk, or `tiles`
+    if constexpr (!kMasked) return tile;
+    while (tile < tiles) {
+      if (tile / kWindow != window) look(tile / kWindow);
+      const uint64_t rest = flags >> (tile % kWindow);
+      if (rest != 0) return min(tile + __builtin_ctzll(rest), tiles);
+      tile = (window + 1) * kWindow;
+    }
+    return tiles;
+  };
+
+  int tile = next_tile(first_tile);
+  if (tile < tiles) {
+    load_tile(tile);
     store_tile(0);
   }
+  // Nothing is in flight when the walk begins (the compiler cannot tell the first products'
+  // operand from the tile asked for meanwhile, and waited for both).
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
   lds_barrier();
-  for (int tile = 0; tile < tiles; ++tile) {
-    const bool more = tile + 1 < tiles;
-    if (more) load_tile(tile + 1);
+  for (int turn = 0; tile < tiles; turn ^= 1) {
+    const int following = next_tile(tile + 1);
+    const bool more = following < tiles;
+    if (more) load_tile(following);
     const int key0 = tile * kTileKeys;
     bool active = first_query < a.length && !(a.causal && key0 > past + first_query + kWaveQueries - 1);
     uint32_t allowed = 0xFFFFFFFFu;
-    if (a.mask != nullptr && active) {
+    if (kMasked && active) {
       const uint8_t* row = a.mask + query_row * a.mask_stride;
       allowed = 0;
 #pragma unroll
-      for (int e = 0; e < 32; ++e) {
-        const int key = key0 + (e / 16) * 32 + 8 * ((e % 16) / 4) + 4 * half + e % 4;
-        allowed |= (row[min(key, a.rows - 1)] != 0 ? 1u : 0u) << e;
+      for (int e = 0; e < 32; e += 4) {   // runs of 4 keys
+        const int key = key0 + (e / 16) * 32 + 8 * ((e % 16) / 4) + 4 * half;
+        const bool whole = key + 4 <= a.rows;
+        const uint32_t word = whole ? mask_word(row + key) : 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t byte = whole ? (word >> (8 * i)) & 0xFFu : key + i < a.rows ? row[key + i] : 0;
+          allowed |= (byte != 0 ? 1u : 0u) << (e + i);
+        }
       }
       active = __ballot(allowed != 0) != 0;
     }
     if (active) {   // the same for the whole wave
-      const uint16_t* tile_k = lds + (tile & 1) * 2 * kTile;
+      const uint16_t* tile_k = lds + turn * 2 * kTile;
       const uint16_t* tile_v = tile_k + kTile;
       f32x16 s[2] = {f32x16{}, f32x16{}};
 #pragma unroll
@@ -242,13 +316,13 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
         }
       }
       const bool edge = key0 + kTileKeys > a.rows ||
-                        (a.causal && key0 + kTileKeys - 1 > past + first_query) || a.mask != nullptr;
+                        (a.causal && key0 + kTileKeys - 1 > past + first_query) || kMasked;
       if (edge) {
         const int bound = a.causal ? min(a.rows - 1, past + query) : a.rows - 1;
 #pragma unroll
         for (int e = 0; e < 32; ++e) {
           const int key = key0 + (e / 16) * 32 + 8 * ((e % 16) / 4) + 4 * half + e % 4;
-          const bool keep = key <= bound && ((allowed >> e) & 1u) != 0;
+          const bool keep = key <= bound && (!kMasked || ((allowed >> e) & 1u) != 0);
           s[e / 16][e % 16] = keep ? s[e / 16][e % 16] : -INFINITY;
         }
       }
@@ -306,14 +380,34 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
       }
       total += (sums[0] + sums[1]) + (sums[2] + sums[3]);
     }
-    if (more) store_tile((tile + 1) & 1);
+    if (more) store_tile(turn ^ 1);
     lds_barrier();
+    tile = following;
   }
 
   uint32_t low, high;
   half_pair(__float_as_uint(total), low, high);
-  const float inverse = 1.0f / (__uint_as_float(low) + __uint_as_float(high));
+  total = __uint_as_float(low) + __uint_as_float(high);
   if (query >= a.length) return;
+  if (a.splits > 1) {
+    const int64_t at = (static_cast<int64_t>(split) * a.heads + head) * a.length + query;
+    float* row = a.partial + at * D + 4 * half;
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        *reinterpret_cast<f32x4*>(row + b * 32 + 8 * i) =
+            f32x4{out[b][4 * i], out[b][4 * i + 1], out[b][4 * i + 2], out[b][4 * i + 3]};
+      }
+    }
+    if (half == 0) {
+      float* state = a.partial + static_cast<int64_t>(a.splits) * a.heads * a.length * D + 2 * at;
+      state[0] = top;
+      state[1] = total;
+    }
+    return;
+  }
+  const float inverse = 1.0f / total;
   uint16_t* row = a.out + (static_cast<int64_t>(head) * a.length + query) * D + 4 * half;
 #pragma unroll
   for (int b = 0; b < kBlocks; ++b) {
@@ -327,8 +421,71 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
   }
 }
 
+// Merges the splits' states: 4 columns a thread.
+template <int D>
+__global__ __launch_bounds__(256) void attention_prefill_combine_kernel(const float* partial, uint16_t* out,
+                                                                        int64_t rows, int splits) {
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t row = item / (D / 4);   // head * length + token
+  if (row >= rows) return;
+  const int column = static_cast<int>(item % (D / 4)) * 4;
+  const float2* states = reinterpret_cast<const float2*>(partial + splits * rows * D);
+  float top = -INFINITY;
+  for (int s = 0; s < splits; ++s) top = fmaxf(top, states[s * rows + row].x);
+  const float base = top == -INFINITY ? 0.0f : top;
+  float total = 0.0f;
+  f32x4 sum = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s) {
+    const float2 state = states[s * rows + row];
+    const f32x4 part = *reinterpret_cast<const f32x4*>(partial + (s * rows + row) * D + column);
+    const float factor = __builtin_amdgcn_exp2f(state.x - base);
+    total = __builtin_fmaf(state.y, factor, total);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] = __builtin_fmaf(part[i], factor, sum[i]);
+  }
+  const float inverse = 1.0f / total;
+  uint2 packed;
+  packed.x = pack_bf16(sum[0] * inverse, sum[1] * inverse);
+  packed.y = pack_bf16(sum[2] * inverse, sum[3] * inverse);
+  *reinterpret_cast<uint2*>(out + row * D + column) = packed;
+}
+
+int64_t head_share(int64_t group) { return group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1; }
+
+int64_t query_blocks(int64_t heads, int64_t group, int64_t length) {
+  const int64_t tile = kWaveQueries * (kWaves / head_share(group));
+  return heads / head_share(group) * ((length + tile - 1) / tile);
+}
+
+// Where the queries' tiles leave CUs without a workgroup, each walks its keys in several, of
+// at least four tiles: 64 tokens after 2,000, 32 heads over 8, D = 128: 72.3 -> 24.4 us; 8
+// after 2,500: 82.9 -> 18.3; 20 after 2,000, 64 over 8, D = 64: 48.3 -> 14.9. Two for every
+// CU cost 1,024 tokens of 32 heads 48.3 us, where one does with 42.5, and two tiles each
+// cost 200 tokens 15.2 us for 12.2.
+int64_t key_splits(int64_t heads, int64_t kv_heads, int64_t length, int64_t rows) {
+  const int64_t blocks = query_blocks(heads, heads / kv_heads, length);
+  if (blocks >= kTargetBlocks) return 1;
+  const int64_t by_blocks = (kTargetBlocks + blocks - 1) / blocks;
+  const int64_t by_tiles = (rows + kTileKeys - 1) / kTileKeys / kMinSplitTiles;
+  const int64_t splits = by_blocks < by_tiles ? by_blocks : by_tiles;
+  return splits < 1 ? 1 : splits > kMaxSplits ? kMaxSplits : splits;
+}
+
 }  // namespace
 }  // namespace omnia
+
+extern "C" int64_t omnia_attention_prefill_workspace_bytes(int64_t heads, int64_t kv_heads, int64_t head_dim,
+                                                           int64_t length, int64_t rows) {
+  using namespace omnia;
+  if ((head_dim != 64 && head_dim != 128) || heads <= 0 || kv_heads <= 0 || heads > 4096 || heads % kv_heads != 0 ||
+      length < 0 || rows < length || rows >= (int64_t{1} << 24)) {
+    return -EINVAL;
+  }
+  if (length == 0) return 0;
+  const int64_t splits = key_splits(heads, kv_heads, length, rows);
+  return splits == 1 ? 0 : splits * heads * length * (head_dim + 2) * static_cast<int64_t>(sizeof(float));
+}
 
 extern "C" int32_t omnia_attention_project(const uint16_t* raw_queries, int64_t query_stride,
                                            const uint16_t* raw_keys, int64_t key_stride,
@@ -382,7 +539,8 @@ extern "C" int32_t omnia_attention_prefill(const uint16_t* queries, const uint16
                                            int64_t key_head_stride, int64_t value_head_stride, int64_t heads,
                                            int64_t kv_heads, int64_t head_dim, int64_t length, int64_t rows,
                                            int32_t causal, const uint8_t* mask, int64_t mask_stride,
-                                           const uint16_t* sinks, float scale, uint16_t* out, hipStream_t stream) {
+                                           const uint16_t* sinks, float scale, void* workspace, int64_t workspace_bytes,
+                                           uint16_t* out, hipStream_t stream) {
   using namespace omnia;
   OMNIA_REQUIRE(head_dim == 64 || head_dim == 128, "attention_prefill: head_dim must be 64 or 128");
   OMNIA_REQUIRE(heads > 0 && kv_heads > 0 && heads <= 4096 && heads % kv_heads == 0,
@@ -397,22 +555,29 @@ extern "C" int32_t omnia_attention_prefill(const uint16_t* queries, const uint16
                     value_head_stride >= rows * head_dim,
                 "attention_prefill: head strides must be multiples of 8 covering the rows");
   OMNIA_REQUIRE(mask == nullptr || mask_stride >= rows, "attention_prefill: the mask must cover the rows");
+  const int64_t need = omnia_attention_prefill_workspace_bytes(heads, kv_heads, head_dim, length, rows);
+  OMNIA_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned16(workspace)),
+                "attention_prefill: workspace too small (omnia_attention_prefill_workspace_bytes) or not aligned");
   int32_t rc = check_device(stream);
   if (rc != 0) return rc;
   const int64_t group = heads / kv_heads;
-  const int64_t share = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-  const int64_t tile = kWaveQueries * (kWaves / share);
-  const int64_t blocks = heads / share * ((length + tile - 1) / tile);
+  const int64_t blocks = query_blocks(heads, group, length);
   OMNIA_REQUIRE(blocks < (int64_t{1} << 31), "attention_prefill: too many tiles");
+  const int64_t splits = key_splits(heads, kv_heads, length, rows);
   constexpr float kLog2e = 1.4426950408889634f;
   PrefillArgs a{queries, keys, values, key_head_stride, value_head_stride, mask, mask_stride, sinks, out,
-                static_cast<int>(heads), static_cast<int>(group), static_cast<int>(share),
-                static_cast<int>(length), static_cast<int>(rows), causal != 0 ? 1 : 0, scale * kLog2e, kLog2e};
-  const dim3 grid(static_cast<unsigned>(blocks));
-  if (head_dim == 64) {
-    attention_prefill_kernel<64><<<grid, 256, 0, stream>>>(a);
-  } else {
-    attention_prefill_kernel<128><<<grid, 256, 0, stream>>>(a);
+                static_cast<float*>(workspace), static_cast<int>(heads), static_cast<int>(group),
+                static_cast<int>(head_share(group)), static_cast<int>(length), static_cast<int>(rows),
+                causal != 0 ? 1 : 0, static_cast<int>(splits), scale * kLog2e, kLog2e};
+  const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(splits));
+  const int64_t merged = heads * length;
+  const dim3 merge_grid(static_cast<unsigned>((merged * (head_dim / 4) + 255) / 256));
+  const auto kernel = head_dim == 64 ? (mask ? attention_prefill_kernel<64, true> : attention_prefill_kernel<64, false>)
+                                     : (mask ? attention_prefill_kernel<128, true> : attention_prefill_kernel<128, false>);
+  kernel<<<grid, 256, 0, stream>>>(a);
+  if (splits > 1) {
+    const auto merge = head_dim == 64 ? attention_prefill_combine_kernel<64> : attention_prefill_combine_kernel<128>;
+    merge<<<merge_grid, 256, 0, stream>>>(a.partial, out, merged, a.splits);
   }
   return launched("attention_prefill");
 }

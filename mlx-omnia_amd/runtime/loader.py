@@ -93,8 +93,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                               _P, _P]),
     "omnia_attention_project": (_I32, [_P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _P, _I64, _I64, _F32, _F32,
                                        _I64, _I64, _I64, _I64, _P, _P, _I64, _P, _I64, _P]),
+    "omnia_attention_prefill_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64]),
     "omnia_attention_prefill": (_I32, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I32, _P, _I64,
-                                       _P, _F32, _P, _P]),
+                                       _P, _F32, _P, _I64, _P, _P]),
     "omnia_embed_atlas": (
         _I32,
         [_P, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _P, _P, _P, _P],

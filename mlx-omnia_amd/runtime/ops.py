@@ -1132,11 +1132,15 @@ def attention_prefill(
                  "attention_prefill: sinks must be contiguous bf16 [heads]")
         tensors.append(sinks)
     _require(on_rocm(*tensors), "attention_prefill: tensors must share one ROCm device")
+    nbytes = library().omnia_attention_prefill_workspace_bytes(heads, kv_heads, head_dim, length, rows)
+    _require(nbytes >= 0, "attention_prefill: geometry not served")
+    workspace = torch.empty(nbytes // 4, dtype=F32, device=queries.device) if nbytes else None
     out = _out(out, queries, (heads, length, head_dim), BF16, "out")
     call("omnia_attention_prefill", queries.data_ptr(), keys.data_ptr(), values.data_ptr(), key_stride,
          value_stride, heads, kv_heads, head_dim, length, rows, int(causal),
          mask.data_ptr() if mask is not None else None, mask_stride,
-         sinks.data_ptr() if sinks is not None else None, float(scale), out.data_ptr(), _stream(queries))
+         sinks.data_ptr() if sinks is not None else None, float(scale),
+         workspace.data_ptr() if workspace is not None else None, nbytes, out.data_ptr(), _stream(queries))
     return out
 
 

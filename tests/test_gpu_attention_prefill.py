@@ -17,6 +17,7 @@ import torch
 from mlx_omnia_amd.kernels.resolve import FALLBACKS
 from mlx_omnia_amd.kernels.attention import AttentionStep, FixedKVCache, KVCache
 from mlx_omnia_amd.kernels.qkv_rope import AngleAtlas, AngleTable
+from mlx_omnia_amd.runtime import ops
 from util import assert_bf16_close, bits_of
 
 pytestmark = pytest.mark.gpu
@@ -87,6 +88,30 @@ def test_sink_prefill_matches_the_core_chain(tokens, past, mask):
     got = layer.check(mask)
     if torch.is_tensor(mask):
         assert not bool(got[0, :, 0].any())
+
+
+@pytest.mark.parametrize("tokens,past,heads,kv_heads,sinks", [
+    (2, 1000, 4, 4, False), (5, 2111, 8, 1, False), (70, 600, 2, 2, False), (3, 900, 8, 2, True),
+    (40, 5000, 16, 2, True),
+])
+@pytest.mark.parametrize("banded", [False, True])
+def test_keys_walked_by_several_workgroups(tokens, past, heads, kv_heads, sinks, banded):
+    """Short prompts over many rows: the splits' states merged, with bands that leave whole
+    splits, whole windows of 64 tiles and whole queries without a row (masks of odd strides)."""
+    print(f"prefill splits H={heads}/{kv_heads} T={tokens} past={past} sinks={sinks} banded={banded}", flush=True)
+    assert ops.library().omnia_attention_prefill_workspace_bytes(
+        heads, kv_heads, 64 if sinks else 128, tokens, past + tokens) > 0
+    layer = Layer(tokens + past, heads, kv_heads, 64 if sinks else 128, past, tokens, sinks=sinks, gains=not sinks)
+    mask = "causal"
+    if banded:
+        query = past + torch.arange(tokens, device="cuda")[:, None]
+        row = torch.arange(past + tokens, device="cuda")[None]
+        wide = torch.zeros((tokens, past + tokens + 5), dtype=torch.bool, device="cuda")
+        wide[:, 3 : 3 + past + tokens] = ((row <= query) & (row > query - 100)) | (row == 7)
+        if sinks:
+            wide[1] = False
+        mask = wide[:, 3 : 3 + past + tokens]
+    layer.check(mask)
 
 
 def test_partial_rotation_factor_and_strided_rows():
