@@ -19,15 +19,14 @@
 //
 // Layout. A workgroup (4 waves) owns one kv head and one chunk of cache rows, a multiple
 // of 128; all `gqa` query heads of that kv head attend through it, so every key and value
-// byte is read once per step. A wave walks blocks of 32 rows. Scores come from
-// v_mfma_f32_16x16x32_bf16 (the query heads as M, 16 cache rows as N, four steps over the
-// 128 dimensions); the running max is uniform over the wave, and the weights pass
-// through LDS to the value layout, where lane c of each 16-lane DPP row holds elements
-// [8c, 8c + 8) of a row and the wave's four DPP rows take rows 4j + 0..3 (one load
-// instruction reads 1 KiB of contiguous values). The four DPP rows' context slices add
-// through permlane swaps, the four waves merge through LDS. With one chunk the
-// workgroup writes the context; with several it writes (max, sum, context) to the
-// workspace and a second kernel merges the chunks of each query head.
+// byte is read once per step. A wave walks blocks of 32 rows, loaded 1 KiB of contiguous
+// rows an instruction (lane c of a 16-lane DPP row holds elements [8c, 8c + 8), the four
+// DPP rows take rows 4j + 0..3) and passed through LDS to the operands of
+// v_mfma_f32_16x16x32_bf16, for the scores and for the context. A lane works for one
+// query head throughout, so its running max and sum are its own registers. The waves
+// merge through LDS. With one chunk the workgroup writes the context; with several it
+// writes (max, sum, context) to the workspace and a second kernel merges the chunks of
+// each query head.
 //
 // The chunk holding the write row computes the new key row itself and reads that row
 // from LDS, never from the cache line it has just written.
@@ -100,40 +99,6 @@ __device__ __forceinline__ StepRows step_rows(const AttnArgs& a, int position) {
   return r;
 }
 __device__ __forceinline__ StepRows step_rows(const AttnArgs& a) { return step_rows(a, *a.position); }
-
-__device__ __forceinline__ float row16_fsum(float v) {
-  v += __uint_as_float(dpp<kRowRor8>(__float_as_uint(v)));
-  v += __uint_as_float(dpp<kRowRor4>(__float_as_uint(v)));
-  v += __uint_as_float(dpp<kRowRor2>(__float_as_uint(v)));
-  v += __uint_as_float(dpp<kRowRor1>(__float_as_uint(v)));
-  return v;
-}
-
-__device__ __forceinline__ float row16_fmax(float v) {
-  v = fmaxf(v, __uint_as_float(dpp<kRowRor8>(__float_as_uint(v))));
-  v = fmaxf(v, __uint_as_float(dpp<kRowRor4>(__float_as_uint(v))));
-  v = fmaxf(v, __uint_as_float(dpp<kRowRor2>(__float_as_uint(v))));
-  v = fmaxf(v, __uint_as_float(dpp<kRowRor1>(__float_as_uint(v))));
-  return v;
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-  v = row16_fmax(v);
-  uint32_t lo, hi;
-  row_pair(__float_as_uint(v), lo, hi);
-  v = fmaxf(__uint_as_float(lo), __uint_as_float(hi));
-  half_pair(__float_as_uint(v), lo, hi);
-  return fmaxf(__uint_as_float(lo), __uint_as_float(hi));
-}
-
-__device__ __forceinline__ float wave_total(float v) {
-  v = row16_fsum(v);
-  uint32_t lo, hi;
-  row_pair(__float_as_uint(v), lo, hi);
-  v = __uint_as_float(lo) + __uint_as_float(hi);
-  half_pair(__float_as_uint(v), lo, hi);
-  return __uint_as_float(lo) + __uint_as_float(hi);
-}
 
 // Merge two online-softmax states (running max m, sum l, context slice o). Both lanes of
 // a swap pair call it with the same (lower, upper) order, so they end bit-identical.
@@ -222,120 +187,111 @@ __device__ __forceinline__ void load_block(const AttnArgs& a, int64_t head_base,
   }
 }
 
-// The uniform running max of head h, picked per lane for the heads 4 drow + i it scores.
-template <int GQA>
-__device__ __forceinline__ float head_value(const float (&x)[GQA], int drow, int i) {
-  float out = x[i < GQA ? i : 0];
-#pragma unroll
-  for (int h = 4; h < GQA; h += 4) {
-    if (drow == h / 4) out = x[h + i];
-  }
-  return out;
-}
+// The wave's online softmax state, per lane: lane (drow, c) works for query head c of the
+// group (columns past the group hold zero queries, their state is dropped) and, of the
+// context, dimensions 16 b + 4 drow + i. The maximum is the same in the head's four lanes,
+// the sum is the lane's own rows'.
+struct HeadState {
+  float m, l;
+  f32x4 o[8];
+};
 
-// One block of 32 rows into the wave's online softmax. Scores: q (A operand: head c,
-// dimensions 32 kk + 8 drow) times the key tile (B operand) on v_mfma_f32_16x16x32_bf16,
-// four steps over the 128 dimensions; the result gives lane (drow, c) the scores of heads
-// 4 drow + i for row c of the tile. The running max is uniform over the wave; the
-// weights p pass through LDS to the value layout, where each lane accumulates its slice.
+// One block of 32 rows into the wave's online softmax. The scores are taken transposed: the
+// key tile as A (row c of 16, dimensions 32 kk + 8 drow), the queries as B (head c) on
+// v_mfma_f32_16x16x32_bf16, so lane (drow, c) gets head c's scores of rows 16 t + 4 drow + i,
+// and its weights are the B operand of o^T = V^T p^T as they stand: k = 8 drow + 4 t + i
+// names row 16 t + 4 drow + i for both operands. V^T comes out of LDS by the transposing
+// read. The weights keep their 24 bits, as three bf16 parts with a product each.
 // MASKED: rows at or past c1 drop out (score -inf, value zero).
-template <int GQA, bool MASKED>
-__device__ __forceinline__ void consume_block(const u32x4 (&kb)[8], u32x4 (&vb)[8],
-                                              const bf16x8 (&qa)[4], float (&m)[GQA],
-                                              float (&lsum)[4], float (&o)[GQA][8],
-                                              float (*p_lds)[4 * ((GQA + 3) / 4)], uint16_t* kt_lds,
-                                              float scale_log2, int b0, int drow, int c, int c1) {
-  constexpr int kPitch = 4 * ((GQA + 3) / 4);
+//
+// Bound by the reads of the cache: 5.6 TB/s at 32768 rows of 8 kv heads. With the context
+// on the vector units (a fused multiply-add per row, head and dimension) they were the
+// bound from 4 heads a group on; four layers' steps, both kernels, 32768 rows: 32/8 heads
+// 120.3 us, now 114.2; 64/8 heads 141.2, now 120.0; 32/4 heads 101.0, now 87.8; one and two
+// heads a group 113.5 and 116.2, now 115.0 and 115.4; 32/8 heads at 500 rows 46.3, now 44.5.
+template <bool MASKED>
+__device__ __forceinline__ void consume_block(const u32x4 (&kb)[8], u32x4 (&vb)[8], const bf16x8 (&qa)[4],
+                                              HeadState& state, uint16_t* tile, float scale_log2, int b0,
+                                              int drow, int c, int c1) {
   // The key block into the wave's LDS tile (rows padded to 272 bytes, so the 16 rows an
-  // operand read touches fall on different banks), read back as the B operand: lane
-  // (drow, c) takes row 16t + c, dimensions 32 kk + 8 drow .. + 8. Loading the operand
-  // layout straight from HBM (16 rows per instruction) measured 32.8 us at 32k rows,
-  // against 32.0 us this way.
+  // operand read touches fall on different banks). Loading the operand layout straight from
+  // HBM (16 rows per instruction) measured 32.8 us at 32k rows, against 32.0 us this way.
 #pragma unroll
-  for (int j = 0; j < 8; ++j) *reinterpret_cast<u32x4*>(kt_lds + (4 * j + drow) * kKeyPitch + 8 * c) = kb[j];
+  for (int j = 0; j < 8; ++j) *reinterpret_cast<u32x4*>(tile + (4 * j + drow) * kKeyPitch + 8 * c) = kb[j];
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  float s[2][4];
+  f32x4 s[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    s[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
-      const u32x4 kt = *reinterpret_cast<const u32x4*>(kt_lds + (16 * t + c) * kKeyPitch + 32 * kk + 8 * drow);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[kk], __builtin_bit_cast(bf16x8, kt), acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      s[t][i] = acc[i] * scale_log2;
-      if constexpr (MASKED) s[t][i] = b0 + 16 * t + c < c1 ? s[t][i] : -INFINITY;
+      const u32x4 kt = *reinterpret_cast<const u32x4*>(tile + (16 * t + c) * kKeyPitch + 32 * kk + 8 * drow);
+      s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kt), qa[kk], s[t], 0, 0, 0);
     }
   }
-  // Block max per head: over the two tiles in the lane, then over the 16 rows (lanes).
-  float bmax[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) bmax[i] = row16_fmax(fmaxf(s[0][i], s[1][i]));
-  float f[GQA];
-#pragma unroll
-  for (int h = 0; h < GQA; ++h) {
-    const float bm = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bmax[h % 4]), 16 * (h / 4)));
-    const float mx = fmaxf(m[h], bm);
-    f[h] = m[h] == mx ? 1.0f : __builtin_amdgcn_exp2f(m[h] - mx);
-    m[h] = mx;
-  }
-  // Weights of the lane's heads for its two rows; partial sums stay per lane.
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float mh = head_value(m, drow, i);
-    const float fh = head_value(f, drow, i);
-    float p0, p1;
-    if constexpr (MASKED) {
-      p0 = s[0][i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s[0][i] - mh);
-      p1 = s[1][i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s[1][i] - mh);
-    } else {
-      p0 = __builtin_amdgcn_exp2f(s[0][i] - mh);
-      p1 = __builtin_amdgcn_exp2f(s[1][i] - mh);
-    }
-    lsum[i] = lsum[i] * fh + (p0 + p1);
-    s[0][i] = p0;
-    s[1][i] = p1;
-  }
-  if (4 * drow < GQA) {
-    *reinterpret_cast<f32x4*>(&p_lds[c][4 * drow]) = f32x4{s[0][0], s[0][1], s[0][2], s[0][3]};
-    *reinterpret_cast<f32x4*>(&p_lds[16 + c][4 * drow]) = f32x4{s[1][0], s[1][1], s[1][2], s[1][3]};
-  }
+  // The value block takes the key block's place once every lane has read that.
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  // Values: rescale, then add p * v for the lane's rows 4j + drow.
-#pragma unroll
-  for (int h = 0; h < GQA; ++h) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[h][e] *= f[h];
-  }
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     if constexpr (MASKED) {
       if (b0 + 4 * j + drow >= c1) vb[j] = u32x4{0u, 0u, 0u, 0u};  // never-written rows
     }
-    float vf[8];
-    unpack8(vb[j], vf);
-    float pw[kPitch];
+    *reinterpret_cast<u32x4*>(tile + (4 * j + drow) * kKeyPitch + 8 * c) = vb[j];
+  }
+  float best = -INFINITY;
 #pragma unroll
-    for (int h4 = 0; h4 < kPitch; h4 += 4) {
-      const f32x4 w4 = *reinterpret_cast<const f32x4*>(&p_lds[4 * j + drow][h4]);
-      pw[h4] = w4[0];
-      pw[h4 + 1] = w4[1];
-      pw[h4 + 2] = w4[2];
-      pw[h4 + 3] = w4[3];
-    }
+  for (int t = 0; t < 2; ++t) {
 #pragma unroll
-    for (int h = 0; h < GQA; ++h) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[h][e] = __builtin_fmaf(pw[h], vf[e], o[h][e]);
+    for (int i = 0; i < 4; ++i) {
+      s[t][i] *= scale_log2;
+      if constexpr (MASKED) s[t][i] = b0 + 16 * t + 4 * drow + i < c1 ? s[t][i] : -INFINITY;
+      best = fmaxf(best, s[t][i]);
     }
   }
-  // The next block overwrites p_lds only after every lane has read this one.
+  uint32_t lo, hi;
+  row_pair(__float_as_uint(best), lo, hi);
+  best = fmaxf(__uint_as_float(lo), __uint_as_float(hi));
+  half_pair(__float_as_uint(best), lo, hi);
+  best = fmaxf(__uint_as_float(lo), __uint_as_float(hi));
+  const float top = fmaxf(state.m, best);
+  const float shrink = state.m == top ? 1.0f : __builtin_amdgcn_exp2f(state.m - top);
+  state.m = top;
+  float p[8];
+  float sum = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float x = s[e / 4][e % 4];
+    p[e] = MASKED && x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(x - top);
+    sum += p[e];
+  }
+  state.l = state.l * shrink + sum;
+  u32x4 parts[3];
+  split_weights(p, parts);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  // The transposing read: of each 16-lane row, lane c brings 4 values of row 4 drow + c / 4
+  // and takes dimension c of the four.
+  const uint16_t* at = tile + (4 * drow + c / 4) * kKeyPitch + 4 * (c % 4);
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    typedef __attribute__((address_space(3))) s16x4* LdsPtr;
+    const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPtr)(at + 16 * b));
+    const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPtr)(at + 16 * kKeyPitch + 16 * b));
+    const bf16x8 v = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) state.o[b][i] *= shrink;
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+      state.o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, __builtin_bit_cast(bf16x8, parts[part]), state.o[b],
+                                                           0, 0, 0);
+    }
+  }
+  // The next block overwrites the tile only after every lane has read this one.
   __builtin_amdgcn_wave_barrier();
 }
 
@@ -346,7 +302,7 @@ __device__ __forceinline__ void consume_block(const u32x4 (&kb)[8], u32x4 (&vb)[
 // per-lane choice between the key and value rows a select of two registers: on the
 // struct it was a vector load of the chosen pointer from the argument segment, waited on
 // before the row's own load.
-template <int GQA, bool SCALED, bool PREFETCH = (GQA <= 4)>
+template <int GQA, bool SCALED>
 __global__ __launch_bounds__(kWaves * kWave) void attention_split_kernel(
     const uint16_t* raw_q, const uint16_t* raw_k, const uint16_t* raw_v, uint16_t* k_cache,
     uint16_t* v_cache, int capacity, int chunk, int max_rows, AttnArgs a) {
@@ -358,12 +314,10 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_split_kernel(
   a.capacity = capacity;
   a.chunk = chunk;
   a.max_rows = max_rows;
-  constexpr int kPitch = 4 * ((GQA + 3) / 4);
   __shared__ u32x4 q_lds[GQA][16];      // the roped queries, bf16 pairs
   __shared__ u32x4 kv_lds[2][16];       // the new key and value rows
   __shared__ float merge_lds[kWaves][GQA][kPartial];
-  __shared__ __align__(16) float p_lds[kWaves][kBlockRows][kPitch];  // a block's weights
-  __shared__ __align__(16) uint16_t kt_lds[kWaves][kBlockRows * kKeyPitch];  // a block's keys
+  __shared__ __align__(16) uint16_t tile_lds[kWaves][kBlockRows * kKeyPitch];  // a block's keys, then values
 
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
@@ -462,7 +416,7 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_split_kernel(
   }
   __syncthreads();
 
-  // The A operand: head c (zero past the group), dimensions 32 kk + 8 drow .. + 8.
+  // The queries' operand: head c (zero past the group), dimensions 32 kk + 8 drow .. + 8.
   bf16x8 qa[4];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) {
@@ -470,20 +424,13 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_split_kernel(
     qa[kk] = __builtin_bit_cast(bf16x8, q);
   }
 
-  float m[GQA], lsum[4], o[GQA][8];
+  HeadState state{-INFINITY, 0.0f, {}};
 #pragma unroll
-  for (int h = 0; h < GQA; ++h) {
-    m[h] = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[h][e] = 0.0f;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) lsum[i] = 0.0f;
+  for (int b = 0; b < 8; ++b) state.o[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  // Blocks of the wave: b0, b0 + 128, ... With PREFETCH (the register budget allows a
-  // second buffer) the next block's loads are issued before the current one is consumed,
-  // the two buffers taking turns. Only the chunk's last, partial block runs the masked
-  // form.
+  // Blocks of the wave: b0, b0 + 128, ... The next block's loads are issued before the
+  // current one is consumed, the two buffers taking turns. Only the chunk's last, partial
+  // block runs the masked form.
   constexpr int kStride = kWaves * kBlockRows;
   auto run = [&](u32x4 (&kb)[8], u32x4 (&vb)[8]) {
     if (writer && rows.write >= b0 && rows.write < b0 + kBlockRows) {
@@ -496,55 +443,36 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_split_kernel(
       }
     }
     if (b0 + kBlockRows <= c1) {
-      consume_block<GQA, false>(kb, vb, qa, m, lsum, o, p_lds[wave], kt_lds[wave], a.scale_log2, b0, drow, c, c1);
+      consume_block<false>(kb, vb, qa, state, tile_lds[wave], a.scale_log2, b0, drow, c, c1);
     } else {
-      consume_block<GQA, true>(kb, vb, qa, m, lsum, o, p_lds[wave], kt_lds[wave], a.scale_log2, b0, drow, c, c1);
+      consume_block<true>(kb, vb, qa, state, tile_lds[wave], a.scale_log2, b0, drow, c, c1);
     }
   };
-  if constexpr (PREFETCH) {
-    u32x4 knext[8], vnext[8];
-    while (b0 < c1) {
-      load_block(a, head_base, b0 + kStride, c1, drow, c, knext, vnext);
-      run(kcur, vcur);
-      b0 += kStride;
-      if (b0 >= c1) break;
-      load_block(a, head_base, b0 + kStride, c1, drow, c, kcur, vcur);
-      run(knext, vnext);
-      b0 += kStride;
-    }
-  } else {
-    for (; b0 < c1; b0 += kStride) {
-      run(kcur, vcur);
-      load_block(a, head_base, b0 + kStride, c1, drow, c, kcur, vcur);
-    }
+  u32x4 knext[8], vnext[8];
+  while (b0 < c1) {
+    load_block(a, head_base, b0 + kStride, c1, drow, c, knext, vnext);
+    run(kcur, vcur);
+    b0 += kStride;
+    if (b0 >= c1) break;
+    load_block(a, head_base, b0 + kStride, c1, drow, c, kcur, vcur);
+    run(knext, vnext);
+    b0 += kStride;
   }
 
-  // The wave's state: the max is uniform already; the sums add over the 16 lanes of each
-  // DPP row (rows of the tiles), the context slices over the four DPP rows.
-  float l[GQA];
+  // The sums add over the head's four lanes.
+  uint32_t lo, hi;
+  row_pair(__float_as_uint(state.l), lo, hi);
+  const float pair = __uint_as_float(lo) + __uint_as_float(hi);
+  half_pair(__float_as_uint(pair), lo, hi);
+  if (c < GQA) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) lsum[i] = row16_fsum(lsum[i]);
+    for (int b = 0; b < 8; ++b) {
 #pragma unroll
-  for (int h = 0; h < GQA; ++h) {
-    l[h] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(lsum[h % 4]), 16 * (h / 4)));
-  }
-#pragma unroll
-  for (int h = 0; h < GQA; ++h) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      uint32_t lo, hi;
-      row_pair(__float_as_uint(o[h][e]), lo, hi);
-      float v = __uint_as_float(lo) + __uint_as_float(hi);
-      half_pair(__float_as_uint(v), lo, hi);
-      o[h][e] = __uint_as_float(lo) + __uint_as_float(hi);
+      for (int i = 0; i < 4; ++i) merge_lds[wave][c][16 * b + 4 * drow + i] = state.o[b][i];
     }
     if (drow == 0) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) merge_lds[wave][h][8 * c + e] = o[h][e];
-      if (c == 0) {
-        merge_lds[wave][h][kD] = m[h];
-        merge_lds[wave][h][kD + 1] = l[h];
-      }
+      merge_lds[wave][c][kD] = state.m;
+      merge_lds[wave][c][kD + 1] = __uint_as_float(lo) + __uint_as_float(hi);
     }
   }
   __syncthreads();

@@ -132,9 +132,9 @@ __device__ __forceinline__ uint32_t mask_word(const uint8_t* at) {
 //
 // Bound by the matrix cores and the softmax's VALU work about equally. The torch chain it
 // replaces wrote and read the fp32 scores five times and widened and repeated K and V:
-// 4,096 tokens, 32 heads over 4, D = 128, causal: 6,181 -> 304 us a call (460 TFLOP/s of the
+// 4,096 tokens, 32 heads over 4, D = 128, causal: 6,181 -> 297 us a call (460 TFLOP/s of the
 // products counted once, twice that on the matrix cores); 777 tokens after 1,500, 64 heads
-// over 8, D = 64, sinks: 1,962 -> 81 us.
+// over 8, D = 64, sinks: 1,962 -> 82 us.
 template <int D, bool kMasked>
 __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a) {
   constexpr int kSteps = D / 16, kBlocks = D / 32, kChunks = D / 8;
@@ -352,18 +352,7 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
           sums[j % 4] += p[j];
         }
         u32x4 parts[3];
-#pragma unroll
-        for (int part = 0; part < 3; ++part) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint32_t packed = pack_bf16(p[2 * j], p[2 * j + 1]);
-            parts[part][j] = packed;
-            if (part < 2) {
-              p[2 * j] -= bf16_lo(packed);
-              p[2 * j + 1] -= bf16_hi(packed);
-            }
-          }
-        }
+        split_weights(p, parts);
 #pragma unroll
         for (int b = 0; b < kBlocks; ++b) {
           typedef __attribute__((address_space(3))) s16x4_lds* LdsPtr;

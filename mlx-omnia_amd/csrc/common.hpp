@@ -127,6 +127,31 @@ __device__ __forceinline__ u32x4 pack8(const float in[8]) {
   return v;
 }
 
+// Eight softmax weights (each zero, or a positive normal number) as three bf16 operands of
+// the matrix unit that add up to their 24 bits: the top half of the number, of what that
+// leaves, and of what is left then, each cut off and not rounded, so that no part is
+// negative. A part of a positive weight is at least the smallest normal number: times an
+// infinite value every part gives that infinity, and not a NaN, as the weight itself would.
+// (Twice 2^-126 is no more than the exponential drops when its result underflows.)
+// Keeping the parts from zero costs a prompt's attention 4%: 285 against 297 us for 4,096
+// tokens of 32 heads.
+__device__ __forceinline__ void split_weights(float (&p)[8], u32x4 (&parts)[3]) {
+#pragma unroll
+  for (int part = 0; part < 3; ++part) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t x0 = __float_as_uint(p[2 * j]);
+      const uint32_t x1 = __float_as_uint(p[2 * j + 1]);
+      parts[part][j] = __builtin_amdgcn_perm(x1, x0, 0x07060302u);
+      if (part < 2) {
+        p[2 * j] = __builtin_amdgcn_fmed3f(p[2 * j] - __uint_as_float(x0 & 0xffff0000u), p[2 * j], 0x1p-126f);
+        p[2 * j + 1] =
+            __builtin_amdgcn_fmed3f(p[2 * j + 1] - __uint_as_float(x1 & 0xffff0000u), p[2 * j + 1], 0x1p-126f);
+      }
+    }
+  }
+}
+
 // Butterfly sum over groups of `width` consecutive lanes (width a power of two <= 64).
 // Every lane of a group ends with the group's total.
 template <int width, typename T>

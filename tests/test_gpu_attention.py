@@ -305,3 +305,20 @@ def test_golden_fixture():
     assert_bf16_close(bits_of(out), golden["out"], min_exact=0.99)
     assert_bf16_close(bits_of(kc)[:, position], golden["key_row"], min_exact=0.999)
     assert np.array_equal(bits_of(vc)[:, position], golden["value_row"])
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(4, 4), (8, 4), (16, 4), (32, 4)])
+@pytest.mark.parametrize("row", [0, 31, 161, 256])
+def test_an_infinite_value_gives_that_infinity(heads, kv_heads, row):
+    # The weights are multiplied in parts: a part that is zero, or of the other sign, would
+    # turn the infinity into a NaN. The other dimensions are as without it.
+    print(f"attention infinite value H={heads} KV={kv_heads} row={row}", flush=True)
+    case = Case(heads, kv_heads, 300, 32, seed=row + heads)
+    want, _, _ = case.run(257)
+    values = case.vc.clone()
+    values[:, row, 5], values[:, row, 77] = float("inf"), float("-inf")
+    got, _, _ = case.run(257, vc=values)
+    got, want = (x.reshape(heads, D) for x in (got, want))
+    assert np.all(got[:, 5] == 0x7F80) and np.all(got[:, 77] == 0xFF80)
+    rest = [d for d in range(D) if d not in (5, 77)]
+    assert np.array_equal(got[:, rest], want[:, rest])

@@ -153,3 +153,17 @@ def test_a_row_that_attends_nothing_is_nan_and_later_rows_are_not_read():
     cache.offset = 0
     again = layer.steps[0](*layer.raw, mask=mask)
     assert np.array_equal(bits_of(got), bits_of(again))
+
+
+@pytest.mark.parametrize("past,tokens", [(0, 70), (300, 5)])
+def test_an_infinite_value_gives_that_infinity(past, tokens):
+    layer = Layer(12, 8, 2, 128, past, tokens)
+    plain = layer.steps[0](*layer.raw, mask=None)
+    layer.caches[0].offset = past
+    raw = [layer.raw[0], layer.raw[1], layer.raw[2].clone()]
+    row = raw[2].view(tokens, -1)[2]
+    row[5], row[77] = float("inf"), float("-inf")      # the first cached head's
+    got = layer.steps[0](*raw, mask=None)
+    rest = [d for d in range(128) if d not in (5, 77)]
+    assert bool((got[:, :4, :, 5] == float("inf")).all()) and bool((got[:, :4, :, 77] == float("-inf")).all())
+    assert torch.equal(got[..., rest], plain[..., rest]) and torch.equal(got[:, 4:], plain[:, 4:])
