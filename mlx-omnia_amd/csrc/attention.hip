@@ -44,6 +44,8 @@ constexpr int kWaves = 4;
 constexpr int kBlockRows = 32;                        // rows per wave iteration
 constexpr int kChunkUnit = kWaves * kBlockRows;       // a chunk is a multiple of 128 rows
 constexpr int kPartial = kD + 2;                      // context slice, max, sum
+constexpr int kWholeRows = 384;                       // up to here a kv head is one workgroup,
+constexpr int kWholeWaves = 8;                        // of eight waves above one chunk unit
 constexpr int kTargetGroups = 512;                    // workgroups a long cache is split into
 constexpr int kMaxSplits = 1024;                      // chunks per kv head at most
 constexpr int kCombineWaves = 16;                     // waves merging one query head
@@ -302,8 +304,8 @@ __device__ __forceinline__ void consume_block(const u32x4 (&kb)[8], u32x4 (&vb)[
 // per-lane choice between the key and value rows a select of two registers: on the
 // struct it was a vector load of the chosen pointer from the argument segment, waited on
 // before the row's own load.
-template <int GQA, bool SCALED>
-__global__ __launch_bounds__(kWaves * kWave) void attention_split_kernel(
+template <int GQA, bool SCALED, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void attention_split_kernel(
     const uint16_t* raw_q, const uint16_t* raw_k, const uint16_t* raw_v, uint16_t* k_cache,
     uint16_t* v_cache, int capacity, int chunk, int max_rows, AttnArgs a) {
   a.raw_q = raw_q;
@@ -316,8 +318,8 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_split_kernel(
   a.max_rows = max_rows;
   __shared__ u32x4 q_lds[GQA][16];      // the roped queries, bf16 pairs
   __shared__ u32x4 kv_lds[2][16];       // the new key and value rows
-  __shared__ float merge_lds[kWaves][GQA][kPartial];
-  __shared__ __align__(16) uint16_t tile_lds[kWaves][kBlockRows * kKeyPitch];  // a block's keys, then values
+  __shared__ float merge_lds[WAVES][GQA][kPartial];
+  __shared__ __align__(16) uint16_t tile_lds[WAVES][kBlockRows * kKeyPitch];  // a block's keys, then values
 
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
@@ -428,10 +430,10 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_split_kernel(
 #pragma unroll
   for (int b = 0; b < 8; ++b) state.o[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  // Blocks of the wave: b0, b0 + 128, ... The next block's loads are issued before the
+  // Blocks of the wave: b0, b0 + 32 WAVES, ... The next block's loads are issued before the
   // current one is consumed, the two buffers taking turns. Only the chunk's last, partial
   // block runs the masked form.
-  constexpr int kStride = kWaves * kBlockRows;
+  constexpr int kStride = WAVES * kBlockRows;
   auto run = [&](u32x4 (&kb)[8], u32x4 (&vb)[8]) {
     if (writer && rows.write >= b0 && rows.write < b0 + kBlockRows) {
 #pragma unroll
@@ -478,13 +480,13 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_split_kernel(
   __syncthreads();
 
   // Merge the four waves (in wave order) and emit: thread t serves elements of the heads.
-  for (int idx = threadIdx.x; idx < GQA * kD; idx += kWaves * kWave) {
+  for (int idx = threadIdx.x; idx < GQA * kD; idx += WAVES * kWave) {
     const int g = idx / kD;
     const int e = idx % kD;
     float mm = merge_lds[0][g][kD], ll = merge_lds[0][g][kD + 1];
     float oo[1] = {merge_lds[0][g][e]};
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) {
+    for (int w = 1; w < WAVES; ++w) {
       const float o2[1] = {merge_lds[w][g][e]};
       merge_state(mm, ll, oo, merge_lds[w][g][kD], merge_lds[w][g][kD + 1], o2);
     }
@@ -585,23 +587,40 @@ __global__ __launch_bounds__(kCombineWaves * kWave) void attention_combine_kerne
   }
 }
 
+// Up to kWholeRows rows one workgroup takes a kv head's whole cache, above 128 rows with
+// eight waves, and there is no second kernel: its launch and its wait for the states (4 us
+// a step) weigh more than the reads that one compute unit then makes alone (about 52 KB/us).
+// Four layers' steps of 32/8 heads, split and merged against whole: 130 rows 40.9 and 29.5
+// us, 250 rows 44.7 and 36.0, 500 rows 44.4 and 45.9, 1020 rows 45.1 and 67.1; 64/8 and 4/4
+// heads cross at the same place. Above, about kTargetGroups workgroups in all.
 int chunk_rows(int max_rows, int kv_heads) {
+  if (max_rows <= kChunkUnit) return kChunkUnit;
   const int per_head = (kTargetGroups + kv_heads - 1) / kv_heads;
+  if (max_rows <= kWholeRows) return kWholeRows;
   int chunk = (max_rows + per_head - 1) / per_head;
   chunk = max(chunk, (max_rows + kMaxSplits - 1) / kMaxSplits);  // bounds the combine loop
   chunk = (chunk + kChunkUnit - 1) / kChunkUnit * kChunkUnit;
   return chunk < kChunkUnit ? kChunkUnit : chunk;
 }
 
-template <int GQA>
-void launch(const AttnArgs& a, hipStream_t stream) {
+template <int GQA, bool SCALED>
+void launch_split(const AttnArgs& a, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(a.splits), static_cast<unsigned>(a.kv_heads));
-  if (a.mscale != 1.0f) {
-    attention_split_kernel<GQA, true><<<grid, kWaves * kWave, 0, stream>>>(
+  if (a.splits == 1 && a.chunk == kWholeRows) {
+    attention_split_kernel<GQA, SCALED, kWholeWaves><<<grid, kWholeWaves * kWave, 0, stream>>>(
         a.raw_q, a.raw_k, a.raw_v, a.k_cache, a.v_cache, a.capacity, a.chunk, a.max_rows, a);
   } else {
-    attention_split_kernel<GQA, false><<<grid, kWaves * kWave, 0, stream>>>(
+    attention_split_kernel<GQA, SCALED, kWaves><<<grid, kWaves * kWave, 0, stream>>>(
         a.raw_q, a.raw_k, a.raw_v, a.k_cache, a.v_cache, a.capacity, a.chunk, a.max_rows, a);
+  }
+}
+
+template <int GQA>
+void launch(const AttnArgs& a, hipStream_t stream) {
+  if (a.mscale != 1.0f) {
+    launch_split<GQA, true>(a, stream);
+  } else {
+    launch_split<GQA, false>(a, stream);
   }
   if (a.splits > 1) {
     attention_combine_kernel<GQA><<<dim3(static_cast<unsigned>(a.kv_heads * GQA)), kCombineWaves * kWave, 0, stream>>>(

@@ -322,3 +322,15 @@ def test_an_infinite_value_gives_that_infinity(heads, kv_heads, row):
     assert np.all(got[:, 5] == 0x7F80) and np.all(got[:, 77] == 0xFF80)
     rest = [d for d in range(D) if d not in (5, 77)]
     assert np.array_equal(got[:, rest], want[:, rest])
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(2, 2), (8, 4), (16, 4), (16, 2)])
+@pytest.mark.parametrize("position", [126, 127, 128, 159, 160, 255, 256, 383, 384, 511])
+def test_one_workgroup_and_split_caches(heads, kv_heads, position):
+    # 1 to 128 rows four waves, to 384 eight waves, above it several workgroups and the merge.
+    print(f"attention H={heads} KV={kv_heads} pos={position}", flush=True)
+    case = Case(heads, kv_heads, 600, 64, seed=position + heads)
+    case.check(position)
+    early = position - 120
+    got, _, _ = case.run(early, max_rows=position + 1)     # a bound above the attended rows
+    assert_bf16_close(got, case.oracle(early)[0], min_exact=0.99)
