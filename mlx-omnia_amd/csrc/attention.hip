@@ -587,20 +587,33 @@ __global__ __launch_bounds__(kCombineWaves * kWave) void attention_combine_kerne
   }
 }
 
+// Rows of a chunk when a cache is split, for about kTargetGroups workgroups in all.
+int split_rows(int max_rows, int kv_heads) {
+  const int per_head = (kTargetGroups + kv_heads - 1) / kv_heads;
+  int chunk = (max_rows + per_head - 1) / per_head;
+  chunk = max(chunk, (max_rows + kMaxSplits - 1) / kMaxSplits);  // bounds the combine loop
+  chunk = (chunk + kChunkUnit - 1) / kChunkUnit * kChunkUnit;
+  return chunk < kChunkUnit ? kChunkUnit : chunk;
+}
+
+// Bytes of chunk states that a step's memory has to hold, as split: a short cache that one
+// workgroup takes asks for them too, so that what a call has to bring depends on its sizes
+// alone and not on where the line between the two forms lies.
+int64_t state_bytes(int64_t max_rows, int64_t heads, int64_t kv_heads) {
+  const int chunk = split_rows(static_cast<int>(max_rows), static_cast<int>(kv_heads));
+  const int64_t splits = (max_rows + chunk - 1) / chunk;
+  return splits > 1 ? splits * heads * kPartial * static_cast<int64_t>(sizeof(float)) : 0;
+}
+
 // Up to kWholeRows rows one workgroup takes a kv head's whole cache, above 128 rows with
 // eight waves, and there is no second kernel: its launch and its wait for the states (4 us
 // a step) weigh more than the reads that one compute unit then makes alone (about 52 KB/us).
 // Four layers' steps of 32/8 heads, split and merged against whole: 130 rows 40.9 and 29.5
 // us, 250 rows 44.7 and 36.0, 500 rows 44.4 and 45.9, 1020 rows 45.1 and 67.1; 64/8 and 4/4
-// heads cross at the same place. Above, about kTargetGroups workgroups in all.
+// heads cross at the same place. Above, the cache is split.
 int chunk_rows(int max_rows, int kv_heads) {
-  if (max_rows <= kChunkUnit) return kChunkUnit;
-  const int per_head = (kTargetGroups + kv_heads - 1) / kv_heads;
-  if (max_rows <= kWholeRows) return kWholeRows;
-  int chunk = (max_rows + per_head - 1) / per_head;
-  chunk = max(chunk, (max_rows + kMaxSplits - 1) / kMaxSplits);  // bounds the combine loop
-  chunk = (chunk + kChunkUnit - 1) / kChunkUnit * kChunkUnit;
-  return chunk < kChunkUnit ? kChunkUnit : chunk;
+  if (max_rows > kChunkUnit && max_rows <= kWholeRows) return kWholeRows;
+  return split_rows(max_rows, kv_heads);
 }
 
 template <int GQA, bool SCALED>
@@ -656,8 +669,8 @@ int32_t attention_decode_checked(
   const int64_t gqa = heads / kv_heads;
   const int chunk = chunk_rows(static_cast<int>(max_rows), static_cast<int>(kv_heads));
   const int splits = static_cast<int>((max_rows + chunk - 1) / chunk);
-  if (splits > 1) {
-    const int64_t need = kv_heads * splits * gqa * kPartial * static_cast<int64_t>(sizeof(float));
+  const int64_t need = state_bytes(max_rows, heads, kv_heads);
+  if (need > 0) {
     OMNIA_REQUIRE(workspace != nullptr && workspace_bytes >= need,
                   "attention_decode: workspace smaller than omnia_attention_workspace_bytes()");
     OMNIA_REQUIRE(aligned16(workspace), "attention_decode: workspace must be 16-byte aligned");
@@ -791,11 +804,7 @@ extern "C" int32_t omnia_attention_decode_noalloc(
                               angle_rows, rotary_pairs, key_cache, value_cache, capacity, window,
                               position, max_rows, heads, kv_heads, head_dim, out);
   if (rc != 0) return rc;
-  const int chunk = chunk_rows(static_cast<int>(max_rows), static_cast<int>(kv_heads));
-  const int64_t splits = (max_rows + chunk - 1) / chunk;
-  const int64_t need = splits > 1 ? kv_heads * splits * (heads / kv_heads) * kPartial *
-                                        static_cast<int64_t>(sizeof(float))
-                                  : 0;
+  const int64_t need = state_bytes(max_rows, heads, kv_heads);
   if (need > kAttentionScratchBytes) {
     return fail(-EINVAL, "attention_decode_noalloc: this step needs " + std::to_string(need) +
                              " bytes of chunk states, above the static scratch of " +

@@ -104,6 +104,25 @@ def test_noalloc_refuses_more_states_than_the_array_holds():
     assert "static scratch" in loader.last_error()
 
 
+@pytest.mark.skipif(torch.cuda.is_available(),
+                    reason="passes placeholder pointers: checked where no GPU can see them")
+@pytest.mark.parametrize("rows", [129, 256, 384, 385])
+def test_a_step_over_several_chunks_needs_its_workspace(rows):
+    """From 129 rows on a step states its chunk states' size, also where one workgroup takes
+    the rows: a workspace missing, short of it by a byte or misaligned is refused."""
+    lib = loader.library()
+    fake = ctypes.c_void_p(1 << 20)  # never dereferenced: the call returns first
+    heads, kv_heads = 32, 8
+    need = ops.attention_workspace_bytes(heads, kv_heads, D, rows)
+    for workspace, size, said in ((None, need, "smaller"), (fake, need - 1, "smaller"),
+                                  (ctypes.c_void_p((1 << 20) + 8), need, "aligned")):
+        rc = lib.omnia_attention_decode(
+            fake, fake, fake, fake, fake, fake, 1024, 64, 1.0, fake, fake, rows, 0, fake, rows,
+            heads, kv_heads, D, D ** -0.5, 1e-6, workspace, size, fake, None)
+        assert rc == -errno.EINVAL
+        assert said in loader.last_error()
+
+
 def test_scratch_size_matches_the_header():
     import re
     from pathlib import Path
