@@ -81,7 +81,7 @@ class AngleAtlas:
         # fp64: the frequencies f_i; fp32: the inverse row base ** (2i / D).
         self.frequencies = torch.from_numpy(np.ascontiguousarray(frequencies)).to(self.device)
         self.atlas = torch.empty((0, 2 * pairs), dtype=torch.float32, device=self.device)
-        self._viewed = self._table = None
+        self._view: tuple[torch.Tensor, AngleTable] | None = None
         self.grow(rows)
 
     @property
@@ -128,9 +128,11 @@ class AngleAtlas:
     def table(self) -> AngleTable:
         """The atlas as it stands, viewed as cosines and sines (the views made once for each
         growth)."""
-        if self._viewed is not self.atlas:
-            self._table, self._viewed = AngleTable.from_atlas(self.atlas), self.atlas
-        return self._table
+        atlas, view = self.atlas, self._view
+        # The pair is stored whole: another thread may grow the atlas meanwhile.
+        if view is None or view[0] is not atlas:
+            view = self._view = atlas, AngleTable.from_atlas(atlas)
+        return view[1]
 
     def __call__(self, offset: int, length: int) -> torch.Tensor:
         """Rows offset .. offset+length-1, cosines then sines (the `Angles` contract)."""
