@@ -22,8 +22,9 @@
 // byte is read once per step. A wave walks blocks of 32 rows, loaded 1 KiB of contiguous
 // rows an instruction (lane c of a 16-lane DPP row holds elements [8c, 8c + 8), the four
 // DPP rows take rows 4j + 0..3) and passed through LDS to the operands of
-// v_mfma_f32_16x16x32_bf16, for the scores and for the context. A lane works for one
-// query head throughout, so its running max and sum are its own registers. The waves
+// v_mfma_f32_16x16x32_bf16, for the scores and, from four heads a group on, for the
+// context: a lane then works for one query head throughout, so its running max and sum are
+// its own registers. One and two heads sum the context on the vector units. The waves
 // merge through LDS. With one chunk the workgroup writes the context; with several it
 // writes (max, sum, context) to the workspace and a second kernel merges the chunks of
 // each query head.
@@ -32,6 +33,7 @@
 // from LDS, never from the cache line it has just written.
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "common.hpp"
 #include "host.hpp"
@@ -46,6 +48,7 @@ constexpr int kChunkUnit = kWaves * kBlockRows;       // a chunk is a multiple o
 constexpr int kPartial = kD + 2;                      // context slice, max, sum
 constexpr int kWholeRows = 384;                       // up to here a kv head is one workgroup,
 constexpr int kWholeWaves = 8;                        // of eight waves above one chunk unit
+constexpr int kVectorHeads = 2;                       // heads a group summed on the vector units
 constexpr int kTargetGroups = 512;                    // workgroups a long cache is split into
 constexpr int kMaxSplits = 1024;                      // chunks per kv head at most
 constexpr int kCombineWaves = 16;                     // waves merging one query head
@@ -101,6 +104,22 @@ __device__ __forceinline__ StepRows step_rows(const AttnArgs& a, int position) {
   return r;
 }
 __device__ __forceinline__ StepRows step_rows(const AttnArgs& a) { return step_rows(a, *a.position); }
+
+__device__ __forceinline__ float row16_fsum(float v) {
+  v += __uint_as_float(dpp<kRowRor8>(__float_as_uint(v)));
+  v += __uint_as_float(dpp<kRowRor4>(__float_as_uint(v)));
+  v += __uint_as_float(dpp<kRowRor2>(__float_as_uint(v)));
+  v += __uint_as_float(dpp<kRowRor1>(__float_as_uint(v)));
+  return v;
+}
+
+__device__ __forceinline__ float row16_fmax(float v) {
+  v = fmaxf(v, __uint_as_float(dpp<kRowRor8>(__float_as_uint(v))));
+  v = fmaxf(v, __uint_as_float(dpp<kRowRor4>(__float_as_uint(v))));
+  v = fmaxf(v, __uint_as_float(dpp<kRowRor2>(__float_as_uint(v))));
+  v = fmaxf(v, __uint_as_float(dpp<kRowRor1>(__float_as_uint(v))));
+  return v;
+}
 
 // Merge two online-softmax states (running max m, sum l, context slice o). Both lanes of
 // a swap pair call it with the same (lower, upper) order, so they end bit-identical.
@@ -210,7 +229,7 @@ struct HeadState {
 // on the vector units (a fused multiply-add per row, head and dimension) they were the
 // bound from 4 heads a group on; four layers' steps, both kernels, 32768 rows: 32/8 heads
 // 120.3 us, now 114.2; 64/8 heads 141.2, now 120.0; 32/4 heads 101.0, now 87.8; one and two
-// heads a group 113.5 and 116.2, now 115.0 and 115.4; 32/8 heads at 500 rows 46.3, now 44.5.
+// heads a group take the vector form below; 32/8 heads at 500 rows 46.3, now 44.5.
 template <bool MASKED>
 __device__ __forceinline__ void consume_block(const u32x4 (&kb)[8], u32x4 (&vb)[8], const bf16x8 (&qa)[4],
                                               HeadState& state, uint16_t* tile, float scale_log2, int b0,
@@ -297,6 +316,96 @@ __device__ __forceinline__ void consume_block(const u32x4 (&kb)[8], u32x4 (&vb)[
   __builtin_amdgcn_wave_barrier();
 }
 
+// The same state for groups of one and two heads, whose context is summed on the vector
+// units: per head, the maximum (uniform over the wave) and dimensions 8 c + e of the lane's
+// rows 4 j + drow; per lane, the sums of heads 4 drow + i over its rows c of the tiles.
+template <int GQA>
+struct VectorState {
+  float m[GQA], l[4], o[GQA][8];
+};
+
+// One block of 32 rows, the context on the vector units. Scores: the queries as A (head c),
+// the key tile as B, so lane (drow, c) gets heads 4 drow + i of row c of a tile (the group's
+// heads in DPP row 0). The weights pass through LDS to the value layout, where a lane adds
+// its own slice of the rows as they were loaded.
+// Up to two heads a group these multiply-adds are fewer than the LDS passes and the three
+// products that the matrix form spends on any group. Four layers' steps, this form and the
+// matrix form (us): 8/8 heads 24.7 and 26.6 at 60 rows, 65.2 and 68.9 at 12,000, 110.6 and
+// 112.2 at 32,768; 16/8 heads 25.8 and 26.4, 39.9 and 41.1 at 500 rows, 68.8 and 69.1 at
+// 12,000, 112.5 and 111.5 at 32,768; 32/8 heads 30.3 and 27.8, 77 and 71, 118 and 113.
+template <int GQA, bool MASKED>
+__device__ __forceinline__ void consume_block(const u32x4 (&kb)[8], u32x4 (&vb)[8], const bf16x8 (&qa)[4],
+                                              VectorState<GQA>& state, uint16_t* tile, f32x4* weights,
+                                              float scale_log2, int b0, int drow, int c, int c1) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) *reinterpret_cast<u32x4*>(tile + (4 * j + drow) * kKeyPitch + 8 * c) = kb[j];
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  f32x4 s[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    s[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const u32x4 kt = *reinterpret_cast<const u32x4*>(tile + (16 * t + c) * kKeyPitch + 32 * kk + 8 * drow);
+      s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[kk], __builtin_bit_cast(bf16x8, kt), s[t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s[t][i] *= scale_log2;
+      if constexpr (MASKED) s[t][i] = b0 + 16 * t + c < c1 ? s[t][i] : -INFINITY;
+    }
+  }
+  // Block max per head: over the two tiles in the lane, then over the 16 rows (lanes).
+  float shrink[GQA];
+#pragma unroll
+  for (int h = 0; h < GQA; ++h) {
+    const float best = __uint_as_float(
+        __builtin_amdgcn_readlane(__float_as_uint(row16_fmax(fmaxf(s[0][h], s[1][h]))), 0));
+    const float top = fmaxf(state.m[h], best);
+    shrink[h] = state.m[h] == top ? 1.0f : __builtin_amdgcn_exp2f(state.m[h] - top);
+    state.m[h] = top;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {   // past the group: computed like head 0, dropped
+    const int h = i < GQA ? i : 0;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      s[t][i] = MASKED && s[t][i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s[t][i] - state.m[h]);
+    }
+    state.l[i] = state.l[i] * shrink[h] + (s[0][i] + s[1][i]);
+  }
+  if (drow == 0) {
+    weights[c] = s[0];
+    weights[16 + c] = s[1];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int h = 0; h < GQA; ++h) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) state.o[h][e] *= shrink[h];
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if constexpr (MASKED) {
+      if (b0 + 4 * j + drow >= c1) vb[j] = u32x4{0u, 0u, 0u, 0u};  // never-written rows
+    }
+    float v[8];
+    unpack8(vb[j], v);
+    const f32x4 p = weights[4 * j + drow];
+#pragma unroll
+    for (int h = 0; h < GQA; ++h) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) state.o[h][e] = __builtin_fmaf(p[h], v[e], state.o[h][e]);
+    }
+  }
+  // The next block overwrites the tile and the weights only after every lane has read these.
+  __builtin_amdgcn_wave_barrier();
+}
+
 // The arguments the first loads need come first, as scalars (copies of AttnArgs fields,
 // which replace the struct's own): gfx950 preloads a kernel's leading scalar and pointer
 // arguments into SGPRs at wave launch, so the prologue rows' and the first cache block's
@@ -319,6 +428,8 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_split_kernel(
   __shared__ u32x4 q_lds[GQA][16];      // the roped queries, bf16 pairs
   __shared__ u32x4 kv_lds[2][16];       // the new key and value rows
   __shared__ float merge_lds[WAVES][GQA][kPartial];
+  constexpr bool kVector = GQA <= kVectorHeads;
+  __shared__ f32x4 weight_lds[kVector ? WAVES : 1][kVector ? kBlockRows : 1];  // a block's weights
   __shared__ __align__(16) uint16_t tile_lds[WAVES][kBlockRows * kKeyPitch];  // a block's keys, then values
 
   const int lane = threadIdx.x % kWave;
@@ -426,9 +537,13 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_split_kernel(
     qa[kk] = __builtin_bit_cast(bf16x8, q);
   }
 
-  HeadState state{-INFINITY, 0.0f, {}};
+  std::conditional_t<kVector, VectorState<GQA>, HeadState> state{};
+  if constexpr (kVector) {
 #pragma unroll
-  for (int b = 0; b < 8; ++b) state.o[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int h = 0; h < GQA; ++h) state.m[h] = -INFINITY;
+  } else {
+    state.m = -INFINITY;
+  }
 
   // Blocks of the wave: b0, b0 + 32 WAVES, ... The next block's loads are issued before the
   // current one is consumed, the two buffers taking turns. Only the chunk's last, partial
@@ -444,7 +559,14 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_split_kernel(
         }
       }
     }
-    if (b0 + kBlockRows <= c1) {
+    if constexpr (kVector) {
+      f32x4* weights = weight_lds[wave];
+      if (b0 + kBlockRows <= c1) {
+        consume_block<GQA, false>(kb, vb, qa, state, tile_lds[wave], weights, a.scale_log2, b0, drow, c, c1);
+      } else {
+        consume_block<GQA, true>(kb, vb, qa, state, tile_lds[wave], weights, a.scale_log2, b0, drow, c, c1);
+      }
+    } else if (b0 + kBlockRows <= c1) {
       consume_block<false>(kb, vb, qa, state, tile_lds[wave], a.scale_log2, b0, drow, c, c1);
     } else {
       consume_block<true>(kb, vb, qa, state, tile_lds[wave], a.scale_log2, b0, drow, c, c1);
@@ -461,20 +583,45 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_split_kernel(
     b0 += kStride;
   }
 
-  // The sums add over the head's four lanes.
-  uint32_t lo, hi;
-  row_pair(__float_as_uint(state.l), lo, hi);
-  const float pair = __uint_as_float(lo) + __uint_as_float(hi);
-  half_pair(__float_as_uint(pair), lo, hi);
-  if (c < GQA) {
+  if constexpr (kVector) {
+    // The sums add over the 16 lanes of DPP row 0, the context slices over the four rows.
 #pragma unroll
-    for (int b = 0; b < 8; ++b) {
+    for (int h = 0; h < GQA; ++h) {
+      const float sum = row16_fsum(state.l[h]);
+      float slice[8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) merge_lds[wave][c][16 * b + 4 * drow + i] = state.o[b][i];
+      for (int e = 0; e < 8; ++e) {
+        uint32_t lo, hi;
+        row_pair(__float_as_uint(state.o[h][e]), lo, hi);
+        const float pair = __uint_as_float(lo) + __uint_as_float(hi);
+        half_pair(__float_as_uint(pair), lo, hi);
+        slice[e] = __uint_as_float(lo) + __uint_as_float(hi);
+      }
+      if (drow == 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) merge_lds[wave][h][8 * c + e] = slice[e];
+        if (c == 0) {
+          merge_lds[wave][h][kD] = state.m[h];
+          merge_lds[wave][h][kD + 1] = sum;
+        }
+      }
     }
-    if (drow == 0) {
-      merge_lds[wave][c][kD] = state.m;
-      merge_lds[wave][c][kD + 1] = __uint_as_float(lo) + __uint_as_float(hi);
+  } else {
+    // The sums add over the head's four lanes.
+    uint32_t lo, hi;
+    row_pair(__float_as_uint(state.l), lo, hi);
+    const float pair = __uint_as_float(lo) + __uint_as_float(hi);
+    half_pair(__float_as_uint(pair), lo, hi);
+    if (c < GQA) {
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) merge_lds[wave][c][16 * b + 4 * drow + i] = state.o[b][i];
+      }
+      if (drow == 0) {
+        merge_lds[wave][c][kD] = state.m;
+        merge_lds[wave][c][kD + 1] = __uint_as_float(lo) + __uint_as_float(hi);
+      }
     }
   }
   __syncthreads();
