@@ -404,13 +404,17 @@ extern "C" int64_t omnia_moe_nvfp4_shared_workspace_bytes(int64_t experts, int64
       hidden >= (int64_t{1} << 24)) {
     return 0;
   }
-  // The per-token kernel takes about 84 ps per row of a slot, this one 11 us plus 64 ps per
+  // On the device the per-token kernel takes about 84 ps per row of a slot, this one 11 us plus 64 ps per
   // row of a matrix that it reads: 512 experts, top-10, hidden 2048: 30.4 against 37.1 us at
   // 16 tokens, 59.2 against 49.3 at 32; 16 experts, top-2, hidden 1024: 7.6 against 11.5 us
   // at 32 tokens, 21.0 against 14.4 at 128.
   const int64_t pairs = tokens * top_k;
   const int64_t matrices = (experts < pairs ? experts : pairs) + 1;
   if ((tokens * (top_k + 1) - matrices * 3 / 4) * hidden < (int64_t{128} << 10)) return 0;
+  // Called outside a graph, three launches and their scratch take the host 38 us and one takes
+  // it 32, so that the per-token kernel stays ahead to about 45 us of its own: 45 against 48
+  // us at 24 tokens of the first shape, 57 against 53 at 32; 36 against 38 at 100 of the second.
+  if (tokens * (top_k + 1) * hidden < (int64_t{640} << 10)) return 0;
   const int64_t pass = pass_tokens(hidden, tokens, top_k);
   return plan_bytes(experts, pass * top_k) + pass * (top_k + 1) * row_stride(hidden) * 2;
 }

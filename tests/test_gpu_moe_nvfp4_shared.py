@@ -175,11 +175,11 @@ def test_golden_fixture():
 
 
 @pytest.mark.parametrize("tokens,top_k,hidden,experts", [
-    (24, 10, 2048, 512),    # about the fewest tokens grouped by expert; most experts idle
-    (300, 4, 100, 60),      # 64 tokens a tile; a short last row tile, 4-byte rows of out
-    (1200, 1, 65, 2),       # odd rows: the scalar epilogue
-    (100, 31, 72, 400),     # the most routed slots, 16 tokens a tile
-    (1500, 2, 64, 600),     # experts without a pair
+    (30, 10, 2048, 512),    # about the fewest tokens grouped by expert; most experts idle
+    (1320, 4, 100, 60),     # 64 tokens a tile; a short last row tile, 4-byte rows of out
+    (5050, 1, 65, 2),       # odd rows: the scalar epilogue
+    (300, 31, 72, 400),     # the most routed slots, 16 tokens a tile
+    (3500, 2, 64, 600),     # experts without a pair
     (150, 8, 1408, 500),    # two row tiles a workgroup, the second past the last row
 ])
 def test_grouped_prompt_matches_oracle(tokens, top_k, hidden, experts):
@@ -190,7 +190,7 @@ def test_grouped_prompt_matches_oracle(tokens, top_k, hidden, experts):
     (every running total is at most S); the bound is three of them in one output."""
     print(f"moe_down_combine_nvfp4_shared grouped tokens={tokens} top_k={top_k} hidden={hidden}", flush=True)
     assert ops.library().omnia_moe_nvfp4_shared_workspace_bytes(experts, hidden, 512, tokens, top_k) > 0
-    case = _case(tokens + top_k, tokens, top_k, hidden, 512, experts, special=tokens == 300, invalid=tokens == 100)
+    case = _case(tokens + top_k, tokens, top_k, hidden, 512, experts, special=hidden == 100, invalid=hidden == 72)
     routed, shared, act, chosen, weights, residual = case
     got, want = _both(case)
     assert float(np.mean(got == want)) >= 0.99
