@@ -6,8 +6,8 @@ write and the attention that `DefaultAttentionStep` runs in torch ops
 `project_served` says whether a call's prologue is one of them, before anything is written:
 plain bf16 tensors of the current ROCm device, head_dim 64 or 128, a cache of this package
 with room, gains and angle rows the kernel can read. A call that autograd, a functorch
-transform, a dispatch mode or a compiler follows stays with the torch ops, which they can
-see through. `mask_served` does the same for the attention's mask.
+transform, a dispatch mode, a tracer or a compiler follows stays with the torch ops, which
+they can see through. `mask_served` does the same for the attention's mask.
 """
 
 from __future__ import annotations
@@ -33,6 +33,8 @@ def plain_call(*tensors: torch.Tensor) -> bool:
     """Ordinary tensors on the current ROCm device, with nothing following the operations
     on them: a kernel may then stand in for torch ops."""
     if torch._C._len_torch_dispatch_stack() or torch.compiler.is_compiling():
+        return False
+    if torch._C._get_tracing_state() is not None:
         return False
     if torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0:
         return False

@@ -1,0 +1,77 @@
+"""Which calls the prefill kernels take, on the CPU: the device gate is held open and the two
+kernels replaced by stand-ins that no tracer, transform or compiler can see into (as the real
+ones), so that a call that one of these follows shows which way it went.
+"""
+
+import importlib
+
+import pytest
+import torch
+
+from mlx_omnia_amd.kernels.attention import DefaultAttentionStep, FixedKVCache, HipAttentionStep
+from mlx_omnia_amd.kernels.qkv_rope import AngleAtlas
+
+route = importlib.import_module("mlx_omnia_amd.kernels.attention.prefill")
+HEADS, KV_HEADS, D, TOKENS = 4, 2, 128, 5
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    """The names of the kernels that were reached."""
+    reached = []
+
+    def project(raw_queries, raw_keys, raw_values, *rest, heads, head_dim, **_):
+        reached.append("project")
+        return torch.zeros((heads, raw_queries.shape[1], head_dim), dtype=torch.bfloat16)
+
+    def attention(queries, keys, values, **_):
+        reached.append("prefill")
+        return torch.zeros(queries.shape, dtype=torch.bfloat16)
+
+    monkeypatch.setattr(route, "hip_device", lambda *tensors: True)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: -1, raising=False)
+    monkeypatch.setattr(route.ops, "attention_project", project)
+    monkeypatch.setattr(route.ops, "attention_prefill", attention)
+    return reached
+
+
+def rows(seed, *shape):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16)
+
+
+def raw_rows(seed):
+    return [rows(seed + i, 1, TOKENS, n * D) for i, n in enumerate((HEADS, KV_HEADS, KV_HEADS))]
+
+
+def layer(*, angles=None, gain=None, past=0, capacity=64):
+    """(the step with the kernels, the Core chain over a cache of its own)"""
+    steps = []
+    angles = angles or AngleAtlas(D // 2, base=1e4, rows=64)
+    gains = (rows(1, D), rows(2, D)) if gain is None else (gain, gain)
+    for _ in range(2):
+        cache = FixedKVCache.empty(KV_HEADS, capacity, D)
+        if past:
+            cache.update_and_fetch(rows(3, 1, KV_HEADS, past, D), rows(4, 1, KV_HEADS, past, D))
+        core = DefaultAttentionStep.build(
+            cache, heads=HEADS, kv_heads=KV_HEADS, head_dim=D, scale=D ** -0.5, dtype=torch.bfloat16,
+            query_weight=gains[0], key_weight=gains[1], eps=1e-6, rotary_pairs=D // 2, mscale=1.0,
+            angles=angles, base=1e4, sinks=None)
+        steps.append(core)
+    core = steps[0]
+    step = HipAttentionStep(core.cache, HEADS, KV_HEADS, core.scale, core.eps, 1.0, core.query_weight,
+                            core.key_weight, torch.empty(0), None, torch.empty(0), core)
+    return step, steps[1]
+
+
+def test_a_plain_call_takes_the_kernels(kernels):
+    step, _ = layer()
+    step(*raw_rows(10), mask="causal")
+    assert kernels == ["project", "prefill"] and step.cache.offset == TOKENS
+
+
+def test_a_traced_call_replays_on_new_inputs(kernels):
+    step, core = layer()
+    traced = torch.jit.trace(lambda *raw: step(*raw, mask="causal"), tuple(raw_rows(10)), check_trace=False)
+    assert kernels == []
+    fresh = raw_rows(20)
+    assert torch.equal(traced(*fresh), core(*fresh, mask="causal"))
