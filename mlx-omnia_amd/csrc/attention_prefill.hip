@@ -116,6 +116,15 @@ __device__ __forceinline__ uint32_t mask_word(const uint8_t* at) {
   return word;
 }
 
+// `rows` rows of D values as a buffer, whose loads check their offset against its bytes and
+// bring zeros past them (below 2^24 rows of 256 bytes: an offset is 32 bits).
+template <int D>
+__device__ __forceinline__ auto row_buffer(const uint16_t* first, int rows) {
+  constexpr int kRawDword = 0x00027000;   // the resource's last word: 32-bit data, no swizzle
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(first), 0, static_cast<uint32_t>(rows) * (2u * D),
+                                           kRawDword);
+}
+
 // A workgroup's four waves take 32 queries each: `share` heads of one kv head (the largest
 // of 1, 2, 4 dividing the group, so that the waves read the same keys), 4 / share runs of
 // queries. It walks the attended rows in tiles of 64 through two LDS buffers, the next
@@ -132,9 +141,9 @@ __device__ __forceinline__ uint32_t mask_word(const uint8_t* at) {
 //
 // Bound by the matrix cores and the softmax's VALU work about equally. The torch chain it
 // replaces wrote and read the fp32 scores five times and widened and repeated K and V:
-// 4,096 tokens, 32 heads over 4, D = 128, causal: 6,181 -> 297 us a call (460 TFLOP/s of the
+// 4,096 tokens, 32 heads over 4, D = 128, causal: 6,181 -> 293 us a call (470 TFLOP/s of the
 // products counted once, twice that on the matrix cores); 777 tokens after 1,500, 64 heads
-// over 8, D = 64, sinks: 1,962 -> 82 us.
+// over 8, D = 64, sinks: 1,962 -> 80 us.
 template <int D, bool kMasked>
 __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a) {
   constexpr int kSteps = D / 16, kBlocks = D / 32, kChunks = D / 8;
@@ -152,7 +161,7 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
   const int tile_index = static_cast<int>(blockIdx.x) / head_groups;
   const int query_tile = a.causal ? tiles_of_queries - 1 - tile_index : tile_index;
   const int head = head_group * a.share + wave % a.share;
-  const int kv_head = head / a.group;
+  const int kv_head = head_group * a.share / a.group;   // of every wave
   const int tile_queries = kWaveQueries * (kWaves / a.share);
   const int first_query = query_tile * tile_queries + (wave / a.share) * kWaveQueries;
   const int query = first_query + column;
@@ -166,8 +175,11 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
   const int split_tiles = (all_tiles + a.splits - 1) / a.splits;
   const int first_tile = split * split_tiles;
   const int tiles = min(first_tile + split_tiles, all_tiles);   // past the last
-  const uint16_t* keys = a.keys + kv_head * a.key_stride;
-  const uint16_t* values = a.values + kv_head * a.value_stride;
+  // Buffers of the head's rows: past the last row a load brings zeros. (The last row again
+  // in their place would do for K, whose scores are masked. For V it would not: it has no
+  // weight, but zero times an infinity is a NaN.)
+  const auto keys = row_buffer<D>(a.keys + kv_head * a.key_stride, a.rows);
+  const auto values = row_buffer<D>(a.values + kv_head * a.value_stride, a.rows);
 
   // Q^T as the B operand: column = query, k = 8 half + j of each 16-wide step.
   s16x8 q[kSteps];
@@ -185,10 +197,10 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
   auto load_tile = [&](int tile) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
-      const int row = min(tile * kTileKeys + (static_cast<int>(threadIdx.x) + 256 * i) / kChunks, a.rows - 1);
-      const int64_t at = static_cast<int64_t>(row) * D + chunk * 8;
-      stage_k[i] = *reinterpret_cast<const u32x4*>(keys + at);
-      stage_v[i] = *reinterpret_cast<const u32x4*>(values + at);
+      const int row = min(tile * kTileKeys + (static_cast<int>(threadIdx.x) + 256 * i) / kChunks, a.rows);
+      const int at = static_cast<int>(static_cast<uint32_t>(row) * (2u * D) + chunk * 16u);   // bytes
+      stage_k[i] = __builtin_amdgcn_raw_buffer_load_b128(keys, at, 0, 0);
+      stage_v[i] = __builtin_amdgcn_raw_buffer_load_b128(values, at, 0, 0);
     }
   };
   auto store_tile = [&](int stage) {

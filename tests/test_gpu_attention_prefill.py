@@ -167,3 +167,21 @@ def test_an_infinite_value_gives_that_infinity(past, tokens):
     rest = [d for d in range(128) if d not in (5, 77)]
     assert bool((got[:, :4, :, 5] == float("inf")).all()) and bool((got[:, :4, :, 77] == float("-inf")).all())
     assert torch.equal(got[..., rest], plain[..., rest]) and torch.equal(got[:, 4:], plain[:, 4:])
+
+
+@pytest.mark.parametrize("past,tokens,d", [(0, 65, 128), (0, 127, 64), (300, 5, 128), (600, 5, 128), (900, 3, 64)])
+def test_an_infinite_value_in_the_last_row(past, tokens, d):
+    """The last tile ends past the last row: what stands there in its place has no part in
+    the products (with one workgroup over the keys and with several)."""
+    print(f"prefill infinite last row D={d} T={tokens} past={past}", flush=True)
+    assert (past + tokens) % 64
+    layer = Layer(13, 8, 2, d, past, tokens, sinks=d == 64, gains=d == 128)
+    plain = layer.steps[0](*layer.raw, mask=None)
+    layer.caches[0].offset = past
+    raw = [layer.raw[0], layer.raw[1], layer.raw[2].clone()]
+    row = raw[2].view(tokens, -1)[-1]
+    row[5], row[d + 40] = float("inf"), float("-inf")      # of either cached head
+    got = layer.steps[0](*raw, mask=None)
+    assert bool((got[:, :4, :, 5] == float("inf")).all()) and bool((got[:, 4:, :, 40] == float("-inf")).all())
+    plain[:, :4, :, 5], plain[:, 4:, :, 40] = float("inf"), float("-inf")
+    assert torch.equal(got, plain)
