@@ -80,9 +80,14 @@ class AngleAtlas:
         self.device = torch.device(device if device is not None else "cpu")
         # fp64: the frequencies f_i; fp32: the inverse row base ** (2i / D).
         self.frequencies = torch.from_numpy(np.ascontiguousarray(frequencies)).to(self.device)
-        self.atlas = torch.empty((0, 2 * pairs), dtype=torch.float32, device=self.device)
-        self._view: tuple[torch.Tensor, AngleTable] | None = None
+        self._hold(torch.empty((0, 2 * pairs), dtype=torch.float32, device=self.device))
         self.grow(rows)
+
+    def _hold(self, atlas: torch.Tensor) -> None:
+        """Take `atlas`, and with it the views that `table` gives out: made here, they are
+        what the atlas is, whatever transform or mode follows the calls that read them."""
+        self._view = atlas, AngleTable.from_atlas(atlas)
+        self.atlas = atlas
 
     @property
     def rows(self) -> int:
@@ -118,7 +123,7 @@ class AngleAtlas:
         if old:
             atlas[:old].copy_(self.atlas)
         self._fill(old, atlas[old:])
-        self.atlas = atlas
+        self._hold(atlas)
 
     def ensure(self, position: int) -> None:
         """Grow, if needed, so that row `position` exists (to twice the rows at least)."""
@@ -126,13 +131,10 @@ class AngleAtlas:
             self.grow(max(2 * self.rows, position + 1))
 
     def table(self) -> AngleTable:
-        """The atlas as it stands, viewed as cosines and sines (the views made once for each
-        growth)."""
-        atlas, view = self.atlas, self._view
-        # The pair is stored whole: another thread may grow the atlas meanwhile.
-        if view is None or view[0] is not atlas:
-            view = self._view = atlas, AngleTable.from_atlas(atlas)
-        return view[1]
+        """The atlas as it stands, viewed as cosines and sines."""
+        atlas, (viewed, table) = self.atlas, self._view
+        # Another thread may grow the atlas meanwhile: the views are those of this one, or new.
+        return table if viewed is atlas else AngleTable.from_atlas(atlas)
 
     def __call__(self, offset: int, length: int) -> torch.Tensor:
         """Rows offset .. offset+length-1, cosines then sines (the `Angles` contract)."""

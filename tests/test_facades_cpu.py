@@ -100,6 +100,30 @@ def test_angle_atlas_on_cpu_matches_oracle_and_grows():
         AngleAtlas(64)
 
 
+@pytest.mark.parametrize("follows", ["grad", "jvp", "fake"])
+def test_angle_atlas_tables_outlive_what_followed_a_call(follows):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from mlx_omnia_amd.kernels.qkv_rope import AngleAtlas
+    atlas = AngleAtlas(8, base=1e4, rows=16)
+    x = torch.ones(8)
+    turned = lambda x: (atlas.table().cos[3] * x).sum()
+    if follows == "grad":
+        assert torch.equal(torch.func.grad(turned)(x), atlas.atlas[3, :8])
+    elif follows == "jvp":
+        assert torch.equal(torch.func.jvp(turned, (x,), (x,))[1], atlas.atlas[3, :8].sum())
+    else:
+        with FakeTensorMode(allow_non_fake_inputs=True):
+            turned(torch.ones(8))
+    table = atlas.table()
+    assert type(table.cos) is type(table.sin) is torch.Tensor
+    assert table.cos.data_ptr() == atlas.atlas.data_ptr()
+    assert torch.equal(torch.cat([table.cos, table.sin], dim=-1), atlas.atlas)
+    atlas.ensure(100)
+    assert atlas.table().cos.data_ptr() == atlas.atlas.data_ptr() and atlas.table().cos.shape[0] == atlas.rows
+    assert torch.equal(table.cos, atlas.table().cos[:16])
+
+
+
 def test_angle_atlas_fp32_order_on_cpu_matches_oracle():
     """Laguna's fp32 op order (models/laguna/layers/attention.py:236-243), on the CPU."""
     from mlx_omnia_amd.kernels.qkv_rope import AngleAtlas
