@@ -89,6 +89,14 @@ class AngleAtlas:
         self._view = atlas, AngleTable.from_atlas(atlas)
         self.atlas = atlas
 
+    def __getstate__(self) -> dict:
+        """Saved and copied without the views, which pickle would turn into rows of their own."""
+        return {name: value for name, value in vars(self).items() if name != "_view"}
+
+    def __setstate__(self, state: dict) -> None:
+        vars(self).update(state)
+        self._hold(self.atlas)
+
     @property
     def rows(self) -> int:
         return self.atlas.shape[0]

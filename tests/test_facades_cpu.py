@@ -123,6 +123,23 @@ def test_angle_atlas_tables_outlive_what_followed_a_call(follows):
     assert torch.equal(table.cos, atlas.table().cos[:16])
 
 
+def test_angle_atlas_is_saved_and_copied_without_its_views():
+    import copy
+    import pickle
+    from mlx_omnia_amd.kernels.qkv_rope import AngleAtlas
+    atlas = AngleAtlas(8, base=1e4, rows=1024)
+    saved = pickle.dumps(atlas)
+    assert len(saved) < 1.1 * atlas.atlas.numel() * 4
+    plain = AngleAtlas.__new__(AngleAtlas)      # as one saved before the views were kept
+    plain.__setstate__({name: value for name, value in vars(atlas).items() if name != "_view"})
+    for other in (pickle.loads(saved), copy.copy(atlas), copy.deepcopy(atlas), plain):
+        assert torch.equal(other.atlas, atlas.atlas)
+        assert other.table().cos.data_ptr() == other.atlas.data_ptr()
+        other.ensure(2000)
+        assert other.table().sin.shape[0] == other.rows > atlas.rows
+
+
+
 
 def test_angle_atlas_fp32_order_on_cpu_matches_oracle():
     """Laguna's fp32 op order (models/laguna/layers/attention.py:236-243), on the CPU."""
