@@ -32,9 +32,10 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 def plain_call(*tensors: torch.Tensor) -> bool:
     """Ordinary tensors on the current ROCm device, with nothing following the operations
     on them: a kernel may then stand in for torch ops."""
-    if torch._C._len_torch_dispatch_stack() or torch.compiler.is_compiling():
+    # First, since a compiler follows the questions below as well.
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None:
         return False
-    if torch._C._get_tracing_state() is not None:
+    if torch._C._len_torch_dispatch_stack():
         return False
     if torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0:
         return False
@@ -74,7 +75,12 @@ def _cache_writable(cache, length: int, kv_heads: int, head_dim: int) -> bool:
 def project_served(core, raw_queries, raw_keys, raw_values) -> bool:
     """Whether `project` computes this call's prologue as `core` (a `DefaultAttentionStep`)
     does."""
-    d = core.head_dim
+    d, cache = core.head_dim, core.cache
+    held = [t for t in (core.query_weight, core.key_weight, core.sinks, getattr(cache, "keys", None),
+                        getattr(cache, "values", None)) if t is not None]
+    # Ahead of the questions about addresses, which a wrapped tensor does not answer.
+    if not plain_call(raw_queries, raw_keys, raw_values, *held):
+        return False
     if raw_queries.dim() != 3 or d not in HEAD_DIMS or core.heads % core.kv_heads:
         return False
     length = raw_queries.shape[1]
@@ -88,11 +94,7 @@ def project_served(core, raw_queries, raw_keys, raw_values) -> bool:
         return False
     if not (_gain_readable(core.query_weight, d) and _gain_readable(core.key_weight, d)):
         return False
-    cache = core.cache
-    if not _cache_writable(cache, length, core.kv_heads, d):
-        return False
-    held = [t for t in (core.query_weight, core.key_weight, core.sinks, cache.keys, cache.values) if t is not None]
-    return plain_call(raw_queries, raw_keys, raw_values, *held)
+    return _cache_writable(cache, length, core.kv_heads, d)
 
 
 def mask_served(mask, length: int, rows: int) -> bool:

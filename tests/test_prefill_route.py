@@ -43,11 +43,11 @@ def raw_rows(seed):
     return [rows(seed + i, 1, TOKENS, n * D) for i, n in enumerate((HEADS, KV_HEADS, KV_HEADS))]
 
 
-def layer(*, angles=None, gain=None, past=0, capacity=64):
+def layer(*, angles=None, query_gain=None, past=0, capacity=64):
     """(the step with the kernels, the Core chain over a cache of its own)"""
     steps = []
     angles = angles or AngleAtlas(D // 2, base=1e4, rows=64)
-    gains = (rows(1, D), rows(2, D)) if gain is None else (gain, gain)
+    gains = (rows(1, D) if query_gain is None else query_gain, rows(2, D))
     for _ in range(2):
         cache = FixedKVCache.empty(KV_HEADS, capacity, D)
         if past:
@@ -75,3 +75,21 @@ def test_a_traced_call_replays_on_new_inputs(kernels):
     assert kernels == []
     fresh = raw_rows(20)
     assert torch.equal(traced(*fresh), core(*fresh, mask="causal"))
+
+
+def test_a_compiled_call_is_one_graph_of_the_core_chain(kernels):
+    step, core = layer()
+    raw = raw_rows(10)
+    compiled = torch.compile(lambda *raw: step(*raw, mask="causal"), backend="eager", fullgraph=True)
+    assert torch.equal(compiled(*raw), core(*raw, mask="causal"))
+    assert kernels == [] and step.cache.offset == TOKENS
+
+
+def test_a_gain_that_a_transform_follows(kernels):
+    raw = raw_rows(10)
+
+    def loss(gain, steps):
+        return layer(query_gain=gain)[steps](*raw, mask="causal").float().square().sum()
+
+    got, want = (torch.func.grad(loss)(rows(1, D), steps) for steps in (0, 1))
+    assert kernels == [] and bool(want.any()) and torch.equal(got, want)
