@@ -117,8 +117,8 @@ def _readable_rows(raw: torch.Tensor) -> torch.Tensor:
 
 
 def _angle_rows(core, length: int, device):
-    """The (cos, sin) rows of this call's positions, or None where the layer rotates
-    nothing or the table holds too few rows."""
+    """The (cos, sin) rows of this call's positions, or None where the kernel cannot read
+    them in place (a table too short among them) or autograd follows them."""
     offset, pairs = core.cache.offset, core.rotary_pairs
     if type(core.angles) is AngleTable:
         cos, sin = core.angles.cos[offset : offset + length], core.angles.sin[offset : offset + length]
@@ -127,8 +127,10 @@ def _angle_rows(core, length: int, device):
         cos, sin = rows[:, :pairs], rows[:, pairs : 2 * pairs]
     else:
         cos, sin = core._angles(offset, length, device)
-    shape = (length, pairs)
+    shape, followed = (length, pairs), torch.is_grad_enabled()
     for rows in (cos, sin):
+        if type(rows) not in _PLAIN or (followed and rows.requires_grad):
+            return None
         if (rows.dtype != torch.float32 or rows.device != device or rows.shape != shape
                 or rows.stride(-1) != 1 or rows.data_ptr() % 16):
             return None
@@ -139,7 +141,7 @@ def _angle_rows(core, length: int, device):
 
 def project(core, raw_queries, raw_keys, raw_values):
     """(queries [heads, T, D], keys, values) as `core.project` gives them, the cache written
-    and advanced; None, with nothing written, where the angle rows cannot be read in place."""
+    and advanced; None, with nothing written, where the angle rows are not for the kernel."""
     length, device = raw_queries.shape[1], raw_queries.device
     angles = None
     if core.rotary_pairs:

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from mlx_omnia_amd.kernels.attention import DefaultAttentionStep, FixedKVCache, HipAttentionStep
-from mlx_omnia_amd.kernels.qkv_rope import AngleAtlas
+from mlx_omnia_amd.kernels.qkv_rope import AngleAtlas, AngleTable
 
 route = importlib.import_module("mlx_omnia_amd.kernels.attention.prefill")
 HEADS, KV_HEADS, D, TOKENS = 4, 2, 128, 5
@@ -93,3 +93,18 @@ def test_a_gain_that_a_transform_follows(kernels):
 
     got, want = (torch.func.grad(loss)(rows(1, D), steps) for steps in (0, 1))
     assert kernels == [] and bool(want.any()) and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("table", ["table", "callable"])
+def test_angles_with_a_gradient(kernels, table):
+    raw = raw_rows(10)
+    theta = torch.arange(64.0)[:, None] * torch.linspace(1.0, 0.1, D // 2)
+    gradients = []
+    for index in (0, 1):
+        scale = torch.ones((), requires_grad=True)
+        cos, sin = torch.cos(theta * scale), torch.sin(theta * scale)
+        angles = (AngleTable(cos, sin) if table == "table"
+                  else lambda offset, length: torch.cat([cos, sin], dim=-1)[offset : offset + length])
+        layer(angles=angles)[index](*raw, mask="causal").float().square().sum().backward()
+        gradients.append(scale.grad)
+    assert kernels == [] and bool(gradients[1] != 0) and torch.equal(*gradients)
