@@ -26,6 +26,7 @@ from ..qkv_rope.kernel import AngleTable
 from .cache import FixedKVCache, KVCache
 
 HEAD_DIMS = (64, 128)
+MAX_HEADS, MAX_ROWS = 4096, 1 << 24   # what the entries take: as many heads, fewer rows
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
@@ -81,7 +82,7 @@ def project_served(core, raw_queries, raw_keys, raw_values) -> bool:
     # Ahead of the questions about addresses, which a wrapped tensor does not answer.
     if not plain_call(raw_queries, raw_keys, raw_values, *held):
         return False
-    if raw_queries.dim() != 3 or d not in HEAD_DIMS or core.heads % core.kv_heads:
+    if raw_queries.dim() != 3 or d not in HEAD_DIMS or core.heads % core.kv_heads or core.heads > MAX_HEADS:
         return False
     length = raw_queries.shape[1]
     rows = (1, length, core.kv_heads * d)
@@ -167,7 +168,8 @@ def prefill(core, raw_queries, raw_keys, raw_values, mask):
     if not 0 < core.scale < math.inf:
         return None
     length = raw_queries.shape[1]
-    if not mask_served(mask, length, core.cache.offset + length):
+    rows = core.cache.offset + length
+    if rows >= MAX_ROWS or not mask_served(mask, length, rows):
         return None
     sinks = core.sinks
     if sinks is not None and (sinks.dtype != torch.bfloat16 or not sinks.is_contiguous()

@@ -108,3 +108,20 @@ def test_angles_with_a_gradient(kernels, table):
         layer(angles=angles)[index](*raw, mask="causal").float().square().sum().backward()
         gradients.append(scale.grad)
     assert kernels == [] and bool(gradients[1] != 0) and torch.equal(*gradients)
+
+
+@pytest.mark.parametrize("heads,capacity", [(8192, 8), (1, 1 << 24)])
+def test_sizes_past_the_kernels_stay_with_the_core_chain(kernels, heads, capacity):
+    """Seen before anything is written: the entries themselves would refuse the attention
+    after the prologue had written the cache."""
+    cache = FixedKVCache(*(torch.empty((1, 1, capacity, 64), dtype=torch.bfloat16) for _ in range(2)),
+                         position=capacity - 2)
+    core = DefaultAttentionStep.build(
+        cache, heads=heads, kv_heads=1, head_dim=64, scale=0.125, dtype=torch.bfloat16, query_weight=None,
+        key_weight=None, eps=1e-6, rotary_pairs=0, mscale=1.0, angles=None, base=1e4, sinks=None)
+    raw = [rows(30, 1, 2, n * 64) for n in (heads, 1, 1)]
+    assert route.prefill(core, *raw, "causal") is None
+    assert kernels == [] and cache.offset == capacity - 2
+    lib = route.ops.library()
+    assert lib.omnia_attention_prefill_workspace_bytes(heads, 1, 64, 2, capacity) < 0
+    assert lib.omnia_attention_prefill_workspace_bytes(min(heads, 4096), 1, 64, 2, capacity - 1) >= 0
