@@ -52,7 +52,8 @@ def plain_call(*tensors: torch.Tensor) -> bool:
 
 def _gain_readable(weight: torch.Tensor | None, head_dim: int) -> bool:
     return weight is None or (weight.dtype == torch.bfloat16 and weight.is_contiguous()
-                              and weight.numel() == head_dim and weight.data_ptr() % 16 == 0)
+                              and weight.numel() == head_dim == weight.shape[-1]
+                              and weight.data_ptr() % 16 == 0)
 
 
 def _cache_writable(cache, length: int, kv_heads: int, head_dim: int) -> bool:

@@ -125,3 +125,14 @@ def test_sizes_past_the_kernels_stay_with_the_core_chain(kernels, heads, capacit
     lib = route.ops.library()
     assert lib.omnia_attention_prefill_workspace_bytes(heads, 1, 64, 2, capacity) < 0
     assert lib.omnia_attention_prefill_workspace_bytes(min(heads, 4096), 1, 64, 2, capacity - 1) >= 0
+
+
+def test_a_gain_of_another_shape_is_refused_as_before(kernels):
+    raw = raw_rows(10)
+    for index in (0, 1):
+        step = layer(query_gain=rows(1, D, 1))[index]
+        with pytest.raises(RuntimeError):     # D values, but not along the head
+            step(*raw, mask="causal")
+    step, core = layer(query_gain=rows(1, 1, D))
+    step(*raw, mask="causal")
+    assert kernels == ["project", "prefill"]
