@@ -490,7 +490,14 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_split_kernel(
     ga[3] = *reinterpret_cast<const f32x4*>(angle + a.pairs + 4);
   }
   const StepRows rows = step_rows(a);
-  if (c0 >= rows.count) return;         // whole workgroup, before any barrier
+  if (c0 >= rows.count) {               // whole workgroup, before any barrier
+    if (a.splits == 1) {                // a position below zero: zeros, as the merge gives them
+      for (int idx = threadIdx.x; idx < GQA * kD; idx += WAVES * kWave) {
+        a.out[static_cast<int64_t>(kvh) * GQA * kD + idx] = 0;
+      }
+    }
+    return;
+  }
   const int c1 = min(c0 + a.chunk, rows.count);
   const bool writer = rows.write >= c0 && rows.write < c1;
   const bool norm_item = is_q || (item == GQA && writer);

@@ -334,3 +334,20 @@ def test_one_workgroup_and_split_caches(heads, kv_heads, position):
     early = position - 120
     got, _, _ = case.run(early, max_rows=position + 1)     # a bound above the attended rows
     assert_bf16_close(got, case.oracle(early)[0], min_exact=0.99)
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(2, 2), (16, 2)])
+@pytest.mark.parametrize("rows", [128, 300, 500])
+def test_a_position_below_zero_attends_nothing(heads, kv_heads, rows):
+    # One workgroup of four waves, one of eight, several and the merge: a context of zeros,
+    # the cache untouched.
+    print(f"attention H={heads} KV={kv_heads} rows={rows} position -1", flush=True)
+    case = Case(heads, kv_heads, 600, 64, seed=rows)
+    keys, values = case.kc.clone(), case.vc.clone()
+    out = torch.full((heads, D), 3.0, dtype=torch.bfloat16, device="cuda")
+    ops.attention_decode(
+        to_device(case.raw_q), to_device(case.raw_k), to_device(case.raw_v), to_device(case.qw), to_device(case.kw),
+        case.atlas_dev, keys, values, torch.tensor([-1], dtype=torch.int32, device="cuda"), heads=heads,
+        kv_heads=kv_heads, max_rows=rows, scale=SCALE, eps=EPS, workspace=case.workspace, out=out)
+    assert not bool(out.any())
+    assert torch.equal(keys, case.kc) and torch.equal(values, case.vc)
