@@ -615,7 +615,7 @@ int64_t omnia_attention_prefill_workspace_bytes(int64_t heads, int64_t kv_heads,
  * in fp32 (the probabilities in full), rounded once to bf16; no sink term with null sinks.
  * causal = 1: query t attends rows <= rows - length + t; a mask ([length, rows] bytes, rows
  * `mask_stride` apart, non-zero attends) is applied as well. A query that attends nothing
- * gives 0 / 0 (0 with a sink). queries, out [heads, length, D]; keys, values: head h, row r
+ * gives 0 / 0 (0 with a finite sink). queries, out [heads, length, D]; keys, values: head h, row r
  * at h * head_stride + r * D. workspace: at least omnia_attention_prefill_workspace_bytes,
  * 16-byte aligned (null where that is 0).
  * Replaces: core/kernels/attention/default.py:132-156 (the attention of the Core chain at

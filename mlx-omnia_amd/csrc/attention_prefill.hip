@@ -8,6 +8,8 @@
 //   rounded once; scores = (q . k) * scale, softmax and probabilities x values in fp32,
 //   the sink logit (if any) in the denominator only, one bf16 rounding at the end.
 // A row that attends nothing gives 0 / 0, as the softmax over -inf alone does there.
+#include <cfloat>
+
 #include "common.hpp"
 #include "host.hpp"
 
@@ -234,8 +236,11 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(PrefillArgs a
 #pragma unroll
   for (int b = 0; b < kBlocks; ++b) out[b] = f32x16{};
   const bool sink = a.sinks != nullptr && split == 0;
-  float top = sink ? bf16_to_f32(a.sinks[head]) * a.sink_log2 : -INFINITY;
-  float total = sink && half == 0 ? 1.0f : 0.0f;
+  const float sink_logit = sink ? bf16_to_f32(a.sinks[head]) : -INFINITY;
+  float top = sink ? fminf(fmaxf(sink_logit * a.sink_log2, -FLT_MAX), FLT_MAX) : -INFINITY;
+  // The sink's own weight: 1, or 0 where it is -inf, or NaN where it is +inf or a NaN. (Its
+  // maximum stays finite, so that it compares and cancels.)
+  float total = half == 0 ? __builtin_amdgcn_exp2f(sink_logit - fmaxf(sink_logit, -FLT_MAX)) : 0.0f;
 
   // With a mask, the tiles in which any of the workgroup's queries attends anything: the
   // masks of 64 tiles at a time are read 256 keys a load, so that the tiles outside a band

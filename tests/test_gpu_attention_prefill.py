@@ -185,3 +185,23 @@ def test_an_infinite_value_in_the_last_row(past, tokens, d):
     assert bool((got[:, :4, :, 5] == float("inf")).all()) and bool((got[:, 4:, :, 40] == float("-inf")).all())
     plain[:, :4, :, 5], plain[:, 4:, :, 40] = float("inf"), float("-inf")
     assert torch.equal(got, plain)
+
+
+@pytest.mark.parametrize("past,tokens", [(0, 40), (900, 3)])
+def test_sinks_that_are_not_finite(past, tokens):
+    """As the softmax over the logits has them: one of -inf has no weight (and a query that
+    attends nothing else no result), one of +inf or NaN leaves no result, a huge one zeros."""
+    print(f"prefill sinks not finite T={tokens} past={past}", flush=True)
+    layer = Layer(14, 8, 2, 64, past, tokens, sinks=True, gains=False)
+    for head, value in ((0, float("-inf")), (1, -3.3e38), (2, 3.3e38), (3, float("inf")), (5, float("nan"))):
+        layer.steps[0].strategy.sinks[head] = value
+    assert layer.steps[1].strategy.sinks.data_ptr() == layer.steps[0].strategy.sinks.data_ptr()
+    mask = torch.ones((tokens, past + tokens), dtype=torch.bool, device="cuda").tril(past)
+    mask[1] = False
+    got, want = (step(*layer.raw, mask=mask) for step in layer.steps)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert bool(want[0, 0, 1].isnan().all()) and bool(want[0, [3, 5]].isnan().all())
+    assert not bool(want[0, 0, 2:].isnan().any()) and not bool(want[0, 2].any())
+    assert not bool(want[0, 1, 1].any())
+    keep = ~want.isnan()
+    assert_bf16_close(bits_of(got[keep]), bits_of(want[keep]), min_exact=0.98)
