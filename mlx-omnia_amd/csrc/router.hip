@@ -956,10 +956,10 @@ __global__ __launch_bounds__(kThreads) void residual_rms_router_kernel(RouterArg
   const int r = wave;
   const int64_t t = first + r;
   const bool active = t < a.rows;  // wave-uniform; inactive waves still meet the barriers
-  const bool emit = a.logits != nullptr;
   const bool sigmoid = a.bias != nullptr;
-  // Every logit exact (no selection on the bounds) when logits or keys are written out.
-  const bool exact_all = emit || (sigmoid && a.keys != nullptr);
+  // Every logit exact (no selection on the bounds) when the keys are written out. (Calls that
+  // write the logits of this hidden size run router_logits_kernel.)
+  const bool exact_all = sigmoid && a.keys != nullptr;
   const float n_norm = row_norm[r];
   uint32_t bits[V], upper[V], keys[V];
   bool unsure[V];
@@ -1034,10 +1034,6 @@ __global__ __launch_bounds__(kThreads) void residual_rms_router_kernel(RouterArg
     for (int v = 0; v < V; ++v) {
       if (need[v]) bits[v] = exact_bits[r * E + lane + v * kWave];
     }
-  }
-  if (emit) {
-#pragma unroll
-    for (int v = 0; v < V; ++v) a.logits[t * E + lane + v * kWave] = static_cast<uint16_t>(bits[v]);
   }
   if (sigmoid) {   // the contenders' ranking (split kernel) would spill registers here
     sigmoid_finish<V>(bits, bias, E, a.k, lane, a.keys, a.indices, a.weights, t);
@@ -1435,7 +1431,8 @@ __global__ __launch_bounds__(kThreads) void residual_rms_router_split_kernel(Rou
   // Phase 3: as in residual_rms_router_kernel, one token per wave (two per walker when
   // the row waves have left); the recomputations go to the walkers.
   constexpr int kTokens = kDefer ? 2 : 1;
-  const bool emit = a.logits != nullptr;
+  // The logits of 256 experts are router_logits_kernel's; those of 128 are above 1,280 rows.
+  const bool emit = kExactAll && E == 128 && a.logits != nullptr;
   const bool sigmoid = a.bias != nullptr;
   // Every logit exact (no selection on the bounds) when logits or keys are written out.
   constexpr bool exact_all = kExactAll;
