@@ -77,3 +77,19 @@ def test_every_logit_is_the_rounded_exact_product(rows, hidden, experts):
             assert torch.equal(same, logits)
             assert torch.equal(ops.sigmoid_topk(logits, bias, 8, emit_keys=True, select=False)[2].view(torch.int32),
                                keys.view(torch.int32))
+
+
+@pytest.mark.parametrize("rows,hidden,experts", [
+    (33, 2048, 128), (300, 2048, 256), (33, 4096, 128), (300, 4096, 256),
+])
+def test_keys_without_the_logits_are_those_of_the_logits(rows, hidden, experts):
+    """The fused kernels, every logit exact in them: the same keys and selection as from the
+    logits written by the other paths."""
+    print(f"router keys alone rows={rows} hidden={hidden} experts={experts}", flush=True)
+    xd, rd, wd, gd = (to_device(v) for v in _inputs(rows, hidden, experts, "outliers", seed=rows + experts))
+    bias = torch.linspace(-0.1, 0.1, experts, device="cuda")
+    want = ops.residual_rms_router_sigmoid(xd, rd, wd, gd, bias, k=8, eps=1e-6, select=True)
+    got = ops.residual_rms_router_sigmoid(xd, rd, wd, gd, bias, k=8, eps=1e-6, emit_logits=False, select=True)
+    assert got[2] is None
+    for ours, theirs in zip(got[:2] + got[3:], want[:2] + want[3:]):
+        assert torch.equal(ours.view(torch.int16), theirs.view(torch.int16))
