@@ -452,7 +452,8 @@ int32_t omnia_moe_down_combine_nvfp4_shared(const uint16_t* act, const uint32_t*
                                             const uint16_t* residual, uint16_t* out, hipStream_t stream);
 
 /* Workspace bytes of omnia_moe_down_combine_nvfp4_shared_grouped: 0 where the per-token
- * entry above serves the call better (few tokens, or a contraction other than 512).
+ * entry above serves the call better, its launch from the host included (few tokens), or
+ * alone (a contraction other than 512).
  * -EINVAL for a bad geometry. Pure; touches no device. */
 int64_t omnia_moe_nvfp4_shared_workspace_bytes(int64_t experts, int64_t hidden, int64_t inner,
                                                int64_t tokens, int64_t top_k);

@@ -203,3 +203,29 @@ def test_grouped_prompt_matches_oracle(tokens, top_k, hidden, experts):
             d = np.abs(x[token, slot] @ nvfp4.dequantize(nvfp4.Stack(routed.weight[e:e + 1], routed.scales[e:e + 1]))[0].T)
             np.add.at(size, token, d * weights[token, slot][:, None])
     assert np.all(np.abs(to_f32(got) - to_f32(want)) <= 3 * 2.0 ** -7 * size)
+
+
+def test_a_prompt_of_more_tokens_than_the_scratch_holds():
+    """d of 1,024 tokens fills the scratch, so the last 9 tokens are a pass of their own: both
+    passes agree with the per-token kernel as the oracle's bound above has it."""
+    tokens, top_k, hidden, experts = 1033, 31, 4096, 40
+    print(f"moe_down_combine_nvfp4_shared grouped in passes tokens={tokens}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    rng = np.random.default_rng(3)
+    routed, shared = _stack(rng, experts, hidden, 512), _stack(rng, 1, hidden, 512)
+    act = torch.randn((tokens, top_k + 1, 512), generator=gen, device="cuda").to(torch.bfloat16)
+    chosen = torch.randint(0, experts, (tokens, top_k), generator=gen, device="cuda").to(torch.int32)
+    weights = torch.rand((tokens, top_k), generator=gen, device="cuda") / top_k
+    residual = torch.randn((tokens, hidden), generator=gen, device="cuda").to(torch.bfloat16)
+    lib = ops.library()
+    size = lambda n: lib.omnia_moe_nvfp4_shared_workspace_bytes(experts, hidden, 512, n, top_k)
+    assert size(1024) == size(tokens) > 1 << 28
+    leaf, one = _leaf(routed), _leaf(nvfp4.Stack(shared.weight[0], shared.scales[0]))
+    got = ops.moe_down_combine_nvfp4_shared(act, leaf, one, chosen, weights, residual)
+    want = torch.empty_like(got)
+    ops.call("omnia_moe_down_combine_nvfp4_shared", act.data_ptr(), leaf.weight.data_ptr(), leaf.scales.data_ptr(),
+             experts, one.weight.data_ptr(), one.scales.data_ptr(), hidden, 512, chosen.data_ptr(),
+             weights.data_ptr(), tokens, top_k, residual.data_ptr(), want.data_ptr(),
+             torch.cuda.current_stream().cuda_stream)
+    same = (got.view(torch.int16) == want.view(torch.int16)).float().mean(dim=1)
+    assert float(same[:1024].mean()) >= 0.99 and float(same[1024:].mean()) >= 0.99
