@@ -43,11 +43,11 @@ def plain_call(*tensors: torch.Tensor) -> bool:
     if torch._C._len_torch_function_stack() and any(
             type(mode) is not DeviceContext for mode in _get_current_function_mode_stack()):
         return False
-    followed = torch.is_grad_enabled()
+    followed, index = torch.is_grad_enabled(), tensors[0].get_device()
     for t in tensors:
-        if type(t) not in _PLAIN or (followed and t.requires_grad):
+        if type(t) not in _PLAIN or t.get_device() != index or (followed and t.requires_grad):
             return False
-    return hip_device(*tensors) and tensors[0].get_device() == torch._C._cuda_getDevice()
+    return hip_device(tensors[0]) and index == torch._C._cuda_getDevice()
 
 
 def _gain_readable(weight: torch.Tensor | None, head_dim: int) -> bool:
@@ -57,19 +57,17 @@ def _gain_readable(weight: torch.Tensor | None, head_dim: int) -> bool:
 
 
 def _cache_writable(cache, length: int, kv_heads: int, head_dim: int) -> bool:
-    """A cache whose rows the prologue may write itself: this package's fixed cache with
-    room, or its growing one, of bf16 rows the kernels read in place."""
-    if type(cache) is FixedKVCache:
-        if cache.offset + length > cache.capacity:
-            return False
-    elif type(cache) is not KVCache:
+    """A cache whose rows the prologue may write itself: a fixed one with room, or a growing
+    one, of bf16 rows the kernels read in place."""
+    if type(cache) is FixedKVCache and cache.offset + length > cache.capacity:
         return False
     for buffer in (cache.keys, cache.values):
         if buffer is None:
             continue
-        if (buffer.dtype != torch.bfloat16 or not buffer.is_contiguous() or buffer.dim() != 4
-                or buffer.shape[0] != 1 or buffer.shape[1] != kv_heads or buffer.shape[3] != head_dim
-                or buffer.data_ptr() % 16 != 0):
+        if buffer.dtype != torch.bfloat16 or buffer.dim() != 4 or not buffer.is_contiguous():
+            return False
+        lead, heads, _, width = buffer.shape
+        if lead != 1 or heads != kv_heads or width != head_dim or buffer.data_ptr() % 16 != 0:
             return False
     return True
 
@@ -78,8 +76,9 @@ def project_served(core, raw_queries, raw_keys, raw_values) -> bool:
     """Whether `project` computes this call's prologue as `core` (a `DefaultAttentionStep`)
     does."""
     d, cache = core.head_dim, core.cache
-    held = [t for t in (core.query_weight, core.key_weight, core.sinks, getattr(cache, "keys", None),
-                        getattr(cache, "values", None)) if t is not None]
+    if type(cache) is not KVCache and type(cache) is not FixedKVCache:
+        return False
+    held = [t for t in (core.query_weight, core.key_weight, core.sinks, cache.keys, cache.values) if t is not None]
     # Ahead of the questions about addresses, which a wrapped tensor does not answer.
     if not plain_call(raw_queries, raw_keys, raw_values, *held):
         return False
