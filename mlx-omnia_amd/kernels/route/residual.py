@@ -92,7 +92,7 @@ class HipResidualRouter(ResidualRouterStrategy):
     def __call__(self, x, projected):
         # Few tokens (decode steps, short prefills) take the library's decode path, which
         # needs the logits written out; more tokens run the one fused dispatch without them.
-        decode = x.numel() // x.shape[-1] <= ops.ROUTER_SELECT_VIA_DECODE_ROWS
+        decode = ops.router_select_via_logits(x.numel() // x.shape[-1], x.shape[-1])
         if self.routing.bias is not None:
             summed, normalized, _, _, indices, weights = ops.residual_rms_router_sigmoid(
                 x.contiguous(), projected.contiguous(), self.norm_weight, self.gate,

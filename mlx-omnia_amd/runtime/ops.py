@@ -431,12 +431,23 @@ def pack_router_weight(router_weight: torch.Tensor) -> PackedRouterWeight:
     return PackedRouterWeight(buffer, int(experts), int(hidden))
 
 
-# A selection-only call up to this many rows is faster with its logits written to a scratch
-# tensor (the library's decode path, or its product path at 256 experts of hidden 4096) than
-# in the fused dispatch: measured on MI355X, 12.3 against 15.1 us at 96 rows of 2048 x 128,
-# 19.7 against 19.8 at 128 of 2048 x 256, 20.4 against 25.2 at 128 of 4096 x 128, even or
-# slower above.
+# A selection-only call up to ROUTER_SELECT_VIA_DECODE_ROWS rows takes the device less time
+# with its logits written to a scratch tensor (the library's decode path, or its product path
+# at 256 experts of hidden 4096) than in the fused dispatch: measured on MI355X, 13.1 against
+# 14.8 us at 96 rows of 2048 x 128, 19.4 against 19.4 at 128 of 2048 x 256, 20.0 against 25.8
+# at 128 of 4096 x 128, even or slower above. Called outside a graph it takes the host 21 us (a
+# tensor and a launch more) where one dispatch takes it 16.5, which at hidden 2048 is more than
+# the device saves: 21.1 against 18.0 us a call at 96 rows of 2048 x 128, 21.2 against 19.2 of
+# 2048 x 256. So there those calls go up to 64 rows only.
 ROUTER_SELECT_VIA_DECODE_ROWS = 128
+ROUTER_SELECT_VIA_DECODE_ROWS_EAGER = 64
+
+
+def router_select_via_logits(rows: int, hidden: int) -> bool:
+    """Whether a selection-only call asks for its logits too."""
+    if rows <= ROUTER_SELECT_VIA_DECODE_ROWS_EAGER or rows > ROUTER_SELECT_VIA_DECODE_ROWS:
+        return rows <= ROUTER_SELECT_VIA_DECODE_ROWS_EAGER
+    return hidden > 2048 or torch.cuda.is_current_stream_capturing()
 
 
 def residual_rms_router(

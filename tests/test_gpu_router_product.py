@@ -12,6 +12,8 @@ import numpy as np
 import pytest
 import torch
 
+from mlx_omnia_amd.kernels.leaf import RMSNormLeaf
+from mlx_omnia_amd.kernels.route import ResidualRouter, Routing
 from mlx_omnia_amd.runtime import ops
 from oracle.activations import f64_to_bf16
 from oracle.bf16 import from_float, to_f32
@@ -93,3 +95,31 @@ def test_keys_without_the_logits_are_those_of_the_logits(rows, hidden, experts):
     assert got[2] is None
     for ours, theirs in zip(got[:2] + got[3:], want[:2] + want[3:]):
         assert torch.equal(ours.view(torch.int16), theirs.view(torch.int16))
+
+
+@pytest.mark.parametrize("hidden", [2048, 4096])
+@pytest.mark.parametrize("rows", [64, 65, 128, 129])
+def test_a_selection_takes_one_dispatch_where_the_host_is_the_bound(monkeypatch, rows, hidden):
+    """Eager calls of hidden 2048 above 64 rows, captured ones and hidden 4096 above 128; the
+    selection is the same bits either way."""
+    print(f"router selection rows={rows} hidden={hidden}", flush=True)
+    asked = []
+    router_of = ops.residual_rms_router
+    monkeypatch.setattr(ops, "residual_rms_router",
+                        lambda *args, **kw: asked.append(kw["emit_logits"]) or router_of(*args, **kw))
+    xd, rd, wd, gd = (to_device(v) for v in _inputs(rows, hidden, 128, "outliers", seed=rows))
+    router = ResidualRouter(RMSNormLeaf(wd, 1e-6), gd, routing=Routing(experts=128, k=8))
+    eager = router(xd, rd)
+    assert asked == [rows <= (64 if hidden == 2048 else 128)]
+    want = router_of(xd, rd, wd, gd, k=8, eps=1e-6, emit_logits=not asked[0])
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        captured = router(xd, rd)
+    assert asked[1] == (rows <= 128)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        for got in (eager, captured):
+            for ours, theirs in zip(got, want[:2] + want[3:]):
+                assert torch.equal(ours.view(torch.int16), theirs.view(torch.int16))
