@@ -452,11 +452,15 @@ int32_t omnia_moe_down_combine_nvfp4_shared(const uint16_t* act, const uint32_t*
                                             const uint16_t* residual, uint16_t* out, hipStream_t stream);
 
 /* Workspace bytes of omnia_moe_down_combine_nvfp4_shared_grouped: 0 where the per-token
- * entry above serves the call better, its launch from the host included (few tokens), or
- * alone (a contraction other than 512).
- * -EINVAL for a bad geometry. Pure; touches no device. */
+ * entry above takes the device less time (few tokens), or alone serves the call (a contraction
+ * other than 512). -EINVAL for a bad geometry. Pure; touches no device. */
 int64_t omnia_moe_nvfp4_shared_workspace_bytes(int64_t experts, int64_t hidden, int64_t inner,
                                                int64_t tokens, int64_t top_k);
+
+/* About what the per-token entry takes the device, in ns, at a contraction of 512: a caller
+ * whose own time for three launches and a workspace is longer does better with that entry's
+ * one. -EINVAL for a bad geometry. Pure; touches no device. */
+int64_t omnia_moe_nvfp4_shared_per_token_ns(int64_t experts, int64_t hidden, int64_t tokens, int64_t top_k);
 
 /* omnia_moe_down_combine_nvfp4_shared over a prompt: the same arguments and results (the
  * fp32 sums in another order) with the tokens grouped by expert, in a caller's workspace of

@@ -18,6 +18,8 @@
 // tokens per expert the products. Top-10 of 512 experts plus the shared one, hidden 2048:
 // 813 -> 97 us at 512 tokens (the stacks' 302 MB: 47 us at a copy's rate; 78 in
 // grouped_down_kernel, 9 in the combine, 7 in the plan), 6,471 -> 385 at 4,096.
+#include <cmath>
+
 #include "common.hpp"
 #include "fp4.hpp"
 #include "host.hpp"
@@ -388,6 +390,31 @@ int64_t pass_tokens(int64_t hidden, int64_t tokens, int64_t top_k) {
   return most < tokens ? (most < 1 ? 1 : most) : tokens;
 }
 
+// What either form takes the device, in us, as fitted to 16 to 512 experts, top-1 to top-31,
+// hidden 1024 and 2048 and 100 thousand to a million rows of slots (tokens x (top_k + 1) x
+// hidden) in a graph: within 9% of the per-token kernel's times and, but for a few, 8% of
+// these kernels'. The per-token kernel takes so long per row of a slot, less with few waves
+// or whole groups of them a workgroup (3, 8, 16 slots), more where the matrices of the chosen
+// experts outgrow the L2s. This one reads each of those matrices once.
+// Top-7 of 16 experts, hidden 1024: 22.0 against 18.3 us at 38 tokens, 16.2 against 16.7 at
+// 25; top-10 of 512, hidden 2048: 37 against 43 at 19, 55 against 53 at 30; top-31 of 512: 54
+// against 73 at 13.
+double chosen_rows(int64_t experts, int64_t hidden, int64_t tokens, int64_t top_k) {
+  const double share = static_cast<double>(tokens) * top_k / experts;
+  return experts * -std::expm1(-share) * hidden;   // as many experts as routes drawn evenly choose
+}
+
+double per_token_us(int64_t experts, int64_t hidden, int64_t tokens, int64_t top_k) {
+  const bool far = chosen_rows(experts, hidden, tokens, top_k) > 80e3;   // 23 MB of codes and scales
+  const double ps = top_k < 3 ? (far ? 49 : 45) : top_k < 8 ? (far ? 59 : 50) : top_k < 16 ? (far ? 68 : 57) : far ? 57 : 52;
+  return 6.5 + ps * 1e-6 * (static_cast<double>(tokens) * (top_k + 1) * hidden);
+}
+
+double grouped_us(int64_t experts, int64_t hidden, int64_t tokens, int64_t top_k) {
+  return 12.5 + 0.5 * top_k + 0.0135 * experts + 52.5e-6 * chosen_rows(experts, hidden, tokens, top_k) +
+         5e-6 * (static_cast<double>(tokens) * (top_k + 1) * hidden);
+}
+
 int64_t plan_bytes(int64_t experts, int64_t pairs) {
   return ((experts + 1 + pairs) * 4 + 15) / 16 * 16;
 }
@@ -404,19 +431,16 @@ extern "C" int64_t omnia_moe_nvfp4_shared_workspace_bytes(int64_t experts, int64
       hidden >= (int64_t{1} << 24)) {
     return 0;
   }
-  // On the device the per-token kernel takes about 84 ps per row of a slot, this one 11 us plus 64 ps per
-  // row of a matrix that it reads: 512 experts, top-10, hidden 2048: 30.4 against 37.1 us at
-  // 16 tokens, 59.2 against 49.3 at 32; 16 experts, top-2, hidden 1024: 7.6 against 11.5 us
-  // at 32 tokens, 21.0 against 14.4 at 128.
-  const int64_t pairs = tokens * top_k;
-  const int64_t matrices = (experts < pairs ? experts : pairs) + 1;
-  if ((tokens * (top_k + 1) - matrices * 3 / 4) * hidden < (int64_t{128} << 10)) return 0;
-  // Called outside a graph, three launches and their scratch take the host 38 us and one takes
-  // it 32, so that the per-token kernel stays ahead to about 45 us of its own: 45 against 48
-  // us at 24 tokens of the first shape, 57 against 53 at 32; 36 against 38 at 100 of the second.
-  if (tokens * (top_k + 1) * hidden < (int64_t{640} << 10)) return 0;
+  if (per_token_us(experts, hidden, tokens, top_k) < grouped_us(experts, hidden, tokens, top_k)) return 0;
   const int64_t pass = pass_tokens(hidden, tokens, top_k);
   return plan_bytes(experts, pass * top_k) + pass * (top_k + 1) * row_stride(hidden) * 2;
+}
+
+extern "C" int64_t omnia_moe_nvfp4_shared_per_token_ns(int64_t experts, int64_t hidden, int64_t tokens,
+                                                       int64_t top_k) {
+  using namespace omnia;
+  if (experts <= 0 || hidden <= 0 || tokens < 0 || top_k < 0) return -EINVAL;
+  return static_cast<int64_t>(1e3 * per_token_us(experts, hidden, tokens, top_k));
 }
 
 extern "C" int32_t omnia_moe_down_combine_nvfp4_shared_grouped(

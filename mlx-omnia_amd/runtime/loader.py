@@ -79,6 +79,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "omnia_moe_down_combine_nvfp4_shared": (_I32, [_P, _P, _P, _I64, _P, _P, _I64, _I64, _P, _P, _I64, _I64, _P,
                                                    _P, _P]),
     "omnia_moe_nvfp4_shared_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64]),
+    "omnia_moe_nvfp4_shared_per_token_ns": (_I64, [_I64, _I64, _I64, _I64]),
     "omnia_moe_down_combine_nvfp4_shared_grouped": (_I32, [_P, _P, _P, _I64, _P, _P, _I64, _I64, _P, _P, _I64, _I64,
                                                            _P, _P, _I64, _P, _P]),
     "omnia_moe_gate_up_nvfp4_ordinal": (_I32, [_P, _P, _P, _I64, _I64, _I64, _P, _I64, _P, _P]),

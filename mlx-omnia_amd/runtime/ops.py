@@ -1371,6 +1371,13 @@ def moe_down_combine_nvfp4(
     return out
 
 
+# Called outside a graph, the grouped form's three launches and their scratch take the host 43.5
+# us and the per-token kernel's one takes it 35.5, so that below this the latter is ahead whatever
+# the device does: top-2 of 16 experts, hidden 1504: 36.1 and 44.8 us at 146 tokens, 46.4 and 45.2
+# at 205; top-7 of 128, hidden 1504: 45.6 and 43.9 at 55.
+_GROUPED_HOST_NS = 45_000
+
+
 def moe_down_combine_nvfp4_shared(
     act: torch.Tensor,
     leaf: Nvfp4Leaf,
@@ -1415,8 +1422,11 @@ def moe_down_combine_nvfp4_shared(
     if not (on_rocm(act, chosen, weights, residual, *leaf.tensors(), *shared.tensors())):
         raise ValueError(f"{name}: tensors must share one ROCm device")
     out = _out(out, act, (tokens, hidden), BF16, "out")
-    nbytes = library().omnia_moe_nvfp4_shared_workspace_bytes(experts, hidden, inner, tokens, top_k)
-    if nbytes > 0:   # a prompt: the tokens grouped by expert, on the matrix cores
+    lib = library()
+    nbytes = lib.omnia_moe_nvfp4_shared_workspace_bytes(experts, hidden, inner, tokens, top_k)
+    if nbytes > 0 and (lib.omnia_moe_nvfp4_shared_per_token_ns(experts, hidden, tokens, top_k) >= _GROUPED_HOST_NS
+                       or torch.cuda.is_current_stream_capturing()):
+        # A prompt: the tokens grouped by expert, on the matrix cores.
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=act.device)
         call("omnia_moe_down_combine_nvfp4_shared_grouped", act.data_ptr(), leaf.weight.data_ptr(),
              leaf.scales.data_ptr(), experts, shared.weight.data_ptr(), shared.scales.data_ptr(), hidden, inner,

@@ -229,3 +229,38 @@ def test_a_prompt_of_more_tokens_than_the_scratch_holds():
              torch.cuda.current_stream().cuda_stream)
     same = (got.view(torch.int16) == want.view(torch.int16)).float().mean(dim=1)
     assert float(same[:1024].mean()) >= 0.99 and float(same[1024:].mean()) >= 0.99
+
+
+@pytest.mark.parametrize("tokens,top_k,hidden,experts", [
+    (1320, 4, 100, 60), (5050, 1, 65, 2), (300, 31, 72, 400), (3500, 2, 64, 600),
+])
+def test_grouped_prompt_below_the_host_line(monkeypatch, tokens, top_k, hidden, experts):
+    """Sizes that an eager call gives to the per-token kernel: grouped all the same."""
+    monkeypatch.setattr(ops, "_GROUPED_HOST_NS", 0)
+    test_grouped_prompt_matches_oracle(tokens, top_k, hidden, experts)
+
+
+@pytest.mark.parametrize("tokens,top_k,hidden,experts,eager,captured", [
+    (146, 2, 1504, 16, False, True),      # the host takes longer than the per-token kernel
+    (30, 10, 2048, 512, True, True),
+    (19, 10, 2048, 512, False, False),    # more matrices than tokens to share them
+    (13, 31, 2048, 512, False, False),
+])
+def test_which_form_takes_a_prompt(monkeypatch, tokens, top_k, hidden, experts, eager, captured):
+    print(f"moe_down_combine_nvfp4_shared form tokens={tokens} top_k={top_k} hidden={hidden}", flush=True)
+    routed, shared, act, chosen, weights, residual = _case(tokens, tokens, top_k, hidden, 512, experts)
+    args = (to_device(act), _leaf(routed), _leaf(nvfp4.Stack(shared.weight[0], shared.scales[0])),
+            torch.from_numpy(chosen).cuda(), torch.from_numpy(weights).cuda(), to_device(residual))
+    called, call = [], ops.call
+    monkeypatch.setattr(ops, "call", lambda name, *rest: called.append(name.endswith("grouped")) or call(name, *rest))
+    first = ops.moe_down_combine_nvfp4_shared(*args)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.moe_down_combine_nvfp4_shared(*args)
+    assert called == [eager, captured]
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        same = float((out.view(torch.int16) == first.view(torch.int16)).float().mean())
+        assert same == 1.0 if eager == captured else same >= 0.99
