@@ -16,8 +16,8 @@
 // The per-token kernel reads a token's 11 matrices anew and multiplies on the vector units:
 // bound by that work, 1.6 us a token. Here the floor is the stacks' bytes, or with many
 // tokens per expert the products. Top-10 of 512 experts plus the shared one, hidden 2048:
-// 813 -> 97 us at 512 tokens (the stacks' 302 MB: 47 us at a copy's rate; 78 in
-// grouped_down_kernel, 9 in the combine, 7 in the plan), 6,471 -> 385 at 4,096.
+// 818 -> 103 us at 512 tokens (the stacks' 302 MB: 47 us at a copy's rate; under tracing 87 in
+// grouped_down_kernel, 9 in the combine, 6 in the plan), 6,471 -> 385 at 4,096.
 #include <cmath>
 
 #include "common.hpp"
